@@ -1,8 +1,10 @@
 // qsim_fft.hip -- FourierTransform{1,2,3}D plans on gfx950 (replaces the
 // cuFFT Z2Z plans of src/FourierTransform.cpp:84-128, 336-360, 495-519 and
 // the KISS/FFTW CPU transforms).  Power-of-two axes up to 4096 (FP64) / 8192
-// (FP32) run the register-resident Stockham kernel; every other length that
-// fits twice in LDS runs the generic mixed-radix kernel.
+// (FP32) run the register-resident Stockham kernel; composite lengths up to
+// 5120 with prime factors of at most 13 run the mixed-radix kernel
+// (qsim_mix_fft.hip); every other length that fits twice in LDS runs the
+// generic kernel.
 #include <cmath>
 #include <map>
 #include <mutex>
@@ -209,6 +211,7 @@ int prepare_axis(FftAxis *a, size_t n, size_t S, size_t nlines, int precision)
     a->p2 = is_p2_supported(n, precision);
     QSIM_TRY(twiddle_table(n ? n : 1, precision, &a->tw));
     if (a->p2) return QSIM_OK;
+    if (mix_plan(n, mix_work(n, nlines), &a->mix)) return QSIM_OK;
     size_t esz = precision == 64 ? sizeof(c128) : sizeof(c64);
     size_t per_line = 2 * n * esz;
     const size_t lds_max = 160 * 1024;
@@ -249,6 +252,7 @@ int run_axis(const FftAxis &a, int precision, bool inv, const void *in, void *ou
     // a length-1 axis is a copy/scale: the generic kernel with no factors
     if (a.n == 1 && in == out && scale == 1.0) return QSIM_OK;
     if (a.p2) return launch_fft_p2(precision, a.n, inv, in, out, a.S, a.nlines, a.tw, scale, s);
+    if (a.mix.n) return launch_fft_mix(a, precision, inv, in, out, scale, s);
     if (a.four) {
         // pass 0: nlines*n1 lines of length n2 (stride n1), in -> tmp
         QSIM_TRY(launch_4s(precision, a.n2, 0, inv, in, a.tmp, 1, a.nlines * a.n1, a.n1, a.tw2,

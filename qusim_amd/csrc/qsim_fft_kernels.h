@@ -277,11 +277,12 @@ __global__ void __launch_bounds__((P2Launch<T, N, LF, FftV<T, N>::V>::THREADS))
 
 // Workgroups are dealt to the 8 XCDs round robin (workgroup b on XCD b % 8).
 // For strided line tiles, give each XCD a contiguous range of tiles so the
-// 128 B rows neighbouring tiles share stay in one L2.
-__device__ __forceinline__ size_t xcd_tile(size_t b, size_t nb)
+// 128 B rows neighbouring tiles share stay in one L2: XCD x starts at
+// x * (nb / 8) + min(x, nb % 8).
+__host__ __device__ __forceinline__ size_t xcd_tile(size_t b, size_t nb)
 {
-    if (nb % 8) return b;
-    return (b % 8) * (nb / 8) + b / 8;
+    const size_t x = b % 8, r = nb % 8;
+    return x * (nb / 8) + (x < r ? x : r) + b / 8;
 }
 
 // ---------------------------------------------------------------------------

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "qsim_fft_kernels.h"
+#include "qsim_mix.h"
 
 namespace qsim {
 
@@ -11,6 +12,7 @@ struct FftAxis {
     size_t S = 1;       // stride between consecutive line elements
     size_t nlines = 1;  // number of lines
     bool p2 = false;    // register-resident power-of-two kernel
+    MixPlan mix{};      // mixed-radix kernel (mix.n != 0)
     int L = 1;          // generic kernel: lines per workgroup
     size_t lds = 0;     // generic kernel: dynamic LDS bytes
     GenFactors gf{};
@@ -28,6 +30,8 @@ bool is_p2_supported(size_t n, int precision);
 int prepare_axis(FftAxis *a, size_t n, size_t S, size_t nlines, int precision);
 // free what prepare_axis allocated (the four-step scratch)
 void release_axis(FftAxis *a);
+int launch_fft_mix(const FftAxis &a, int precision, bool inv, const void *in, void *out,
+                   double scale, hipStream_t s);
 // Transform every line of the axis, in -> out, multiplying by `scale`.
 int run_axis(const FftAxis &a, int precision, bool inv, const void *in, void *out, double scale,
              hipStream_t s);

@@ -11,8 +11,10 @@
 // with E_T = Tx Ty separable and 1/(nx ny) folded into Tx.  The first sweep
 // only applies E_V then FFT_y; the last only IFFT_y then E_V.
 // 1D (power-of-two): one workgroup per job keeps psi in registers for all
-// steps.  Other sizes and the infinite-wall boundary run the reference's op
-// sequence unfused (FFT plans + pointwise kernels).
+// steps.  Composite lengths with prime factors of at most 13 run the same
+// schedule on mixed-radix lines (qsim_mix_split.hip), the infinite wall as its
+// odd extension; other sizes run the reference's op sequence unfused (FFT
+// plans + pointwise kernels).
 //
 // Precision 64: complex128 everywhere.  Precision 32 (FP32-mixed): psi is
 // stored and transformed in complex64; every phase factor and inter-pass
@@ -28,28 +30,9 @@
 
 #include "qsim_fft_kernels.h"
 #include "qsim_fft_plan.h"
+#include "qsim_mix_split.h"
 
 namespace qsim {
-
-enum { SW_FIRST = 0, SW_MID = 1, SW_LAST = 2 };
-
-// Device-side description of one job (the kernels index a table of these by
-// blockIdx.y, so many same-shape jobs share one launch).
-struct SplitDev {
-    c128 *psi;             // caller's complex128 state
-    void *work;            // working state (== psi for precision 64)
-    const c128 *ev[4];     // potential factors over the grid
-    const c128 *kx[2];     // kinetic factor along x (2D) or the whole line (1D)
-    const c128 *ky[2];     // kinetic factor along y (2D)
-};
-
-// v * f with f an FP64 factor.  FP32 data is widened, multiplied in FP64 and
-// rounded once, so a near-identity factor (tiny V dt) keeps its sub-ulp part
-// instead of losing it the same way at every step.  A float-float product
-// that rounded v * hi before adding v * lo lost it: at 2048^2, dt = 0.1, that
-// bias was half of a 1.1e-5 psi error after 1000 steps.
-__device__ __forceinline__ c128 apply(c128 v, c128 f) { return v * f; }
-__device__ __forceinline__ c64 apply(c64 v, c128 f) { return cvt<float>(cvt<double>(v) * f); }
 
 template <typename TO, typename TI>
 __device__ __forceinline__ cx<TO> conv(cx<TI> a)
@@ -589,14 +572,6 @@ __global__ void __launch_bounds__((P2Launch<T, N, true, V>::THREADS))
 }
 
 // ---------------------------------------------------------------- 1D job
-// Phase program: start with ev[ev0]; each step runs (kinetic k[i], potential
-// ev[e[i]]) for i < nph; the last potential factor of the last step is
-// ev[ev_end] instead.
-struct Prog1D {
-    int ev0, ev_end, nph;
-    int k[3], e[3];
-};
-
 // Radix plan of the persistent 1D kernel per length.  A job is one workgroup
 // stepping its line on its own, so each step's chain of dependent work sets
 // the time: lengths 1024, 2048 and 4096 take four-pass plans with 8 elements
@@ -745,6 +720,10 @@ struct qsim_split_job {
     // phase program
     int ev_start = 0, ev_end = 0, nph = 0;
     int ph_k[3] = {0, 0, 0}, ph_e[3] = {0, 0, 0};
+    // mixed-radix lines (FP64): the fused schedule on lengths that are not a
+    // power of two; a 1D infinite wall runs as its odd extension of 2 nx points
+    bool mix = false;
+    MixPlan mix_x{}, mix_y{};
     // unfused path
     qsim_fft_plan *fwd = nullptr, *inv = nullptr;
     c128 *tmp = nullptr, *tmp2 = nullptr;
@@ -787,6 +766,22 @@ int build_ev(qsim_split_job *j, c128 **out, double t, const double *Vre, const d
         ev[i] = cexp(z);
     }));
     *out = ev;
+    return QSIM_OK;
+}
+
+// A wall job's factor table over its odd extension: t[i] = a[i] for
+// 0 < i < n, mirrored above n, zero at the walls 0 and n.
+int extend_wall(qsim_split_job *j, const c128 **table, hipStream_t s)
+{
+    const size_t n = j->d.nx;
+    const c128 *a = *table;
+    void *p;
+    QSIM_TRY(dalloc(j, &p, 2 * n * sizeof(c128)));
+    c128 *t = (c128 *)p;
+    QSIM_TRY(each(2 * n, s, [=] __device__(size_t i) {
+        t[i] = i == 0 || i == n ? mk(0.0, 0.0) : a[i < n ? i : 2 * n - i];
+    }));
+    *table = t;
     return QSIM_OK;
 }
 
@@ -1172,6 +1167,37 @@ int fused_steps(qsim_split_job *j, const SplitDev *jobs, int njobs, size_t nstep
     return QSIM_OK;
 }
 
+// The same schedule on mixed-radix lines.  It replaces the unfused order where
+// the lengths allow it: one launch for all steps of a 1D job, two sweeps of
+// psi per 2D step instead of eight passes.
+int mix_steps(qsim_split_job *j, size_t nsteps, hipStream_t s)
+{
+    if (j->d.dim == 1) {
+        Prog1D p;
+        p.ev0 = j->ev_start;
+        p.ev_end = j->ev_end;
+        p.nph = j->nph;
+        for (int i = 0; i < 3; ++i) {
+            p.k[i] = j->ph_k[i];
+            p.e[i] = j->ph_e[i];
+        }
+        return mix_run_1d(j->host, p, nsteps, j->mix_x, j->d.nx, j->tw_x, s);
+    }
+    auto row = [&](int mode, int iev, bool twice) {
+        return mix_row_sweep(mode, j->host, j->d.nx, iev, twice, j->mix_y, j->tw_y, s);
+    };
+    QSIM_TRY(row(SW_FIRST, j->ev_start, false));
+    for (size_t st = 0; st < nsteps; ++st)
+        for (int ph = 0; ph < j->nph; ++ph) {
+            QSIM_TRY(mix_col_sweep(j->host, j->d.ny, j->ph_k[ph], j->mix_x, j->tw_x, s));
+            const bool last = st + 1 == nsteps && ph + 1 == j->nph;
+            // between steps the closing and the opening half step meet
+            QSIM_TRY(last ? row(SW_LAST, j->ev_end, false)
+                          : row(SW_MID, j->ph_e[ph], ph + 1 == j->nph));
+        }
+    return QSIM_OK;
+}
+
 // ------------------------------------------------- unfused reference order
 // ExpV: psi *= ev (src/SplittingMethod2D.cpp:81-94); ExpT: FFT, *= E_T, IFFT,
 // *1/N (:96-121).  1D InfiniteWall: src/SplittingMethod1D.cpp:62-81.
@@ -1284,6 +1310,11 @@ int create(qsim_split_job *j, const double *Vre, const double *Vim)
         return set_error(QSIM_ERR_UNSUPPORTED,
                          "FP32-mixed split job needs power-of-two axes (2D: 64..8192, 1D: "
                          "64..16384) and a periodic boundary");
+    if (!j->fused) {
+        const size_t mx = d.boundary == 1 ? 2 * d.nx : d.nx;
+        j->mix = mix_plan(mx, mix_work(mx, d.dim == 1 ? 256 : d.ny), &j->mix_x) &&
+                 (d.dim == 1 || mix_plan(d.ny, mix_work(d.ny, d.nx), &j->mix_y));
+    }
     // potential factors
     SplitDev &h = j->host;
     h.psi = j->psi;
@@ -1299,7 +1330,7 @@ int create(qsim_split_job *j, const double *Vre, const double *Vim)
         j->ev_end = 0;
         j->nph = 1;
         j->ph_k[0] = 0;
-        j->ph_e[0] = 1;
+        j->ph_e[0] = j->mix ? 0 : 1;  // mix: the half step's factor, applied twice
     } else {
         QSIM_TRY(build_ev(j, &ev0, c.C1, Vre, Vim, s));
         QSIM_TRY(build_ev(j, &ev1, c.C2, Vre, Vim, s));
@@ -1317,7 +1348,7 @@ int create(qsim_split_job *j, const double *Vre, const double *Vim)
         j->ph_k[1] = 1;  // D2
         j->ph_e[1] = 1;  // C2
         j->ph_k[2] = 0;  // D1
-        j->ph_e[2] = 2;  // 2 C1 (merged across steps)
+        j->ph_e[2] = j->mix ? 0 : 2;  // 2 C1 (merged across steps)
     }
     // kinetic factors
     const double Dkx = 2 * M_PI / (dx * d.nx);
@@ -1330,11 +1361,12 @@ int create(qsim_split_job *j, const double *Vre, const double *Vim)
         const cd alpha = cd(-0.0, -1.0) * dt / d.hbar;  // src/SplittingMethod2D.cpp:63
         for (int k = 0; k < nk; ++k) {
             c128 *tx, *ty;
-            QSIM_TRY(build_axis(j, &tx, d.nx, alpha * coef[k], DTx, 1.0 / (double)j->n));
+            QSIM_TRY(build_axis(j, &tx, d.nx, alpha * coef[k], DTx,
+                                j->mix ? 1.0 : 1.0 / (double)j->n));
             QSIM_TRY(build_axis(j, &ty, d.ny, alpha * coef[k], DTy, 1.0));
             h.kx[k] = tx;
             h.ky[k] = ty;
-            if (!j->fused) {  // full E_T for the unfused order
+            if (!j->fused && !j->mix) {  // full E_T for the unfused order
                 void *p;
                 QSIM_TRY(dalloc(j, &p, j->n * sizeof(c128)));
                 c128 *et = (c128 *)p;
@@ -1373,9 +1405,20 @@ int create(qsim_split_job *j, const double *Vre, const double *Vim)
             QSIM_TRY(dalloc(j, &p, d.nx * sizeof(c128)));
             QSIM_HIP(hipMemcpy(p, hv.data(), d.nx * sizeof(c128), hipMemcpyHostToDevice));
             j->et_full[k] = (c128 *)p;
+            if (j->mix) {
+                h.kx[k] = j->et_full[k];
+                QSIM_TRY(extend_wall(j, &h.kx[k], s));
+            }
         }
+        if (j->mix)
+            for (const c128 *&ev : h.ev)
+                if (ev) QSIM_TRY(extend_wall(j, &ev, s));
     }
-    if (j->fused) {
+    if (j->mix) {
+        h.work = j->psi;
+        QSIM_TRY(twiddle_table(j->mix_x.n, 64, &j->tw_x));
+        if (d.dim == 2) QSIM_TRY(twiddle_table(d.ny, 64, &j->tw_y));
+    } else if (j->fused) {
         if (d.precision == 32) {
             void *p;
             QSIM_TRY(dalloc(j, &p, j->n * sizeof(c64)));
@@ -1459,6 +1502,7 @@ int qsim_hip_split_steps(qsim_split_job *j, size_t nsteps, qsim_stream_t stream)
     QSIM_CHECK(j, "null job");
     if (nsteps == 0) return QSIM_OK;
     hipStream_t s = as_stream(stream);
+    if (j->mix) return mix_steps(j, nsteps, s);
     if (!j->fused) return unfused_steps(j, nsteps, s);
     if (!j->use_graph || j->d.dim != 2) return fused_steps(j, j->dev, 1, nsteps, s);
     // the sweep sequence of `nsteps` steps is captured once into a HIP graph

@@ -1,0 +1,72 @@
+"""Mixed-radix lines on the GPU: the transform plan against numpy, the
+split-operator jobs against the FP64 oracle, at the edges of their ranges
+(the shortest and longest lengths, one and several lines per workgroup, every
+radix, more butterflies than threads, tiles that the last lines do not fill)."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+from test_gpu_split import gauss2d, run_1d, run_2d
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(4,), (6,), (9,), (15,), (1000,), (3003,), (5000,), (5103,), (5120,), (4900,),
+          (4, 6), (6, 1000), (1000, 6), (100, 169), (143, 77), (1500, 1100), (1, 60), (60, 1),
+          (9, 10, 12), (14, 15, 98), (100, 120, 90), (17, 60, 50)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("precision", [64, 32])
+def test_fft_mixed_radix(shape, precision):
+    """Each axis of at most 6 passes rounds to a few units per pass: 32 units
+    of 2^-53 (FP64) or, with every pass stored in FP32, 2^-24 per pass and
+    axis."""
+    from qusim_amd import fftn
+    rng = np.random.default_rng(len(shape) * 1000 + shape[0])
+    x = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    if precision == 32:
+        x = x.astype(np.complex64)
+    tol = len(shape) * (32 * 2.0 ** -53 if precision == 64 else 6 * 2.0 ** -24)
+    xd = x.astype(np.complex128)
+    assert rel_l2(fftn(x, precision=precision), np.fft.fftn(xd)) < tol
+    assert rel_l2(fftn(x, inverse=True, precision=precision), np.fft.ifftn(xd) * x.size) < tol
+
+
+@pytest.mark.parametrize("n", [4, 12, 60, 1000, 1300, 3003, 5082, 5103, 5120])
+@pytest.mark.parametrize("method", [2, 4])
+def test_1d_mixed_radix_matches_oracle(n, method, oracle):
+    x = -25.0 + 50.0 / n * np.arange(n)
+    psi = np.exp(0.7j * x - (x + 6) ** 2 / 9.0)
+    V = 0.4 * np.exp(-x ** 2 / 6) - 0.02j * np.exp(-(x - 8) ** 2 / 20)
+    e = run_1d(psi, V, -25.0, 25.0, 0.04, 31, method, complex_v=True)
+    ref = oracle.split1d(psi, V, -25.0, 25.0, 0.04, 31, method=method, complex_v=True)
+    assert rel_l2(e.GetPsi(), ref) < 1e-12
+    # steps split over several calls
+    f = run_1d(psi, V, -25.0, 25.0, 0.04, 30, method, complex_v=True, batch=5)
+    f.steps(0)
+    g = oracle.split1d(psi, V, -25.0, 25.0, 0.04, 30, method=method, complex_v=True)
+    assert rel_l2(f.GetPsi(), g) < 1e-12
+
+
+@pytest.mark.parametrize("n", [2, 15, 500, 1024, 1500, 2560])
+@pytest.mark.parametrize("method", [2, 4])
+def test_wall_mixed_radix_matches_oracle(n, method, oracle):
+    """the odd extension to 2n points; psi(0) is not zero at the start"""
+    x = -25.0 + 50.0 / n * np.arange(n)
+    psi = np.exp(0.7j * x - (x + 6) ** 2 / 40.0)
+    V = 0.4 * np.exp(-x ** 2 / 6)
+    e = run_1d(psi, V, -25.0, 25.0, 0.04, 23, method, boundary=1)
+    ref = oracle.split1d(psi, V, -25.0, 25.0, 0.04, 23, method=method, boundary=1)
+    assert rel_l2(e.GetPsi(), ref) < 1e-12
+
+
+@pytest.mark.parametrize("shape", [(4, 4), (6, 1000), (1000, 6), (65, 130), (750, 600),
+                                   (1024, 250), (98, 2048), (5120, 12), (32, 32)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("method", [2, 4])
+def test_2d_mixed_radix_matches_oracle(shape, method, oracle):
+    psi, V, L0, L1 = gauss2d(*shape)
+    got = run_2d(psi, V, L0, L1, 0.05, 6, method, complex_v=True).GetPsi()
+    ref = oracle.split2d(psi, V, L0[0], L0[1], L1[0], L1[1], 0.05, 6, method=method,
+                         complex_v=True)
+    assert rel_l2(got, ref) < 1e-12

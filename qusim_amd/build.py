@@ -20,6 +20,7 @@ HIP_SOURCES = [
     "qsim_split.hip",
     "qsim_born.hip",
     "qsim_gen.hip",
+    "qsim_mix_born.hip",
     "qsim_mix_fft.hip",
     "qsim_mix_split.hip",
 ]

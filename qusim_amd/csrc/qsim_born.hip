@@ -16,7 +16,9 @@
 //   outer sweep (axis 0, strided lines): FFT_x, G0 multiply, IFFT_x.
 // psi0 = e^{i k.r} and the absorbing layer (src/Perburbation.h:150-177) are
 // separable, so both come from per-axis tables instead of grid arrays; the
-// physical V is stored once for all energies.
+// physical V is stored once for all energies.  Grids whose axes are composite
+// lengths with prime factors of at most 13 run the same passes on mixed-radix
+// lines (qsim_mix_born.hip, complex128); other grids the reference's order.
 //
 // Precision 64: complex128 iterates.  Precision 32: complex64 iterates with
 // FP64 V, FP64 phase/absorber tables and FP64 residual sums.
@@ -26,84 +28,10 @@
 
 #include "qsim_fft_kernels.h"
 #include "qsim_fft_plan.h"
+#include "qsim_mix_born.h"
 #include "qsim_reduce.h"
 
 namespace qsim {
-
-enum { BA_START = 0, BA_END = 1, BA_BOTH = 2 };
-enum { PRE_IDENTITY = 0, PRE_VELLEKOOP = 1, PRE_HAO1 = 2, PRE_HAO2 = 3, PRE_NAIVE = 4 };
-
-struct BornGeom {
-    int dim;
-    size_t n0, n1, n2;   // n2 = 1 for 2D
-    size_t ninner;       // length of the last axis
-    size_t nmid;         // 3D: n1; 2D: 1
-};
-
-// per-energy device descriptor
-struct BornDev {
-    void *dpsi;
-    void *tmp;
-    const c128 *pw[3];     // plane-wave factor per axis: exp(i k_a x_a)
-    const double *ab[3];   // absorbing-layer Im V per axis (zeros when naive)
-    double E, eps, slow, inv_n;
-    double inv_eps;        // 1 / eps (0 when eps is 0)
-    double a[3];           // (2 pi hbar / (d n))^2 / 2m per axis
-    double *resid;         // per-block residual partial sums [2 * nblocks]
-};
-
-// potential with the absorbing layer, in the reference's summation order
-__device__ __forceinline__ c128 v_eff(c128 v, const BornDev &J, int dim, size_t i, size_t j,
-                                      size_t k)
-{
-    const double a = dim == 3 ? (ld_g(J.ab[0] + i) + ld_g(J.ab[1] + j)) + ld_g(J.ab[2] + k)
-                              : ld_g(J.ab[0] + i) + ld_g(J.ab[1] + j);
-    return mk(v.x, v.y + a);
-}
-
-__device__ __forceinline__ c128 psi0_at(const BornDev &J, int dim, size_t i, size_t j, size_t k)
-{
-    return dim == 3 ? (ld_g(J.pw[0] + i) * ld_g(J.pw[1] + j)) * ld_g(J.pw[2] + k)
-                    : ld_g(J.pw[0] + i) * ld_g(J.pw[1] + j);
-}
-
-// gamma of op_Vellekoop / op_Hao1 / op_Hao2 (src/DeviceTemplate.h:1020-1077)
-// with the divisions by eps done as products with 1/eps: within an ulp of the
-// quotient, without two FP64 divide sequences per point in the fused sweeps.
-// op_Hao2's 2 / w, w = 1 + i v / eps = (1 - v.y / eps, v.x / eps), is taken
-// as 2 conj(w) / |w|^2 with one real divide instead of a complex division
-// (|w|^2 >= 1 for the absorbing potentials, Im v <= 0, so the unscaled form
-// neither overflows nor underflows); that also frees the registers the
-// merged plane pass needs.
-template <int PRE>
-__device__ __forceinline__ c128 gamma_fused(c128 v, double slow, double eps, double inv_eps)
-{
-    if constexpr (PRE == PRE_VELLEKOOP) {
-        const c128 iv = imul(v);
-        return mk(1. - iv.x * inv_eps, -iv.y * inv_eps) * slow;
-    } else if constexpr (PRE == PRE_HAO1) {
-        const c128 iv = imul(mk(v.x, -v.y));
-        return mk(1. - iv.x * inv_eps, -iv.y * inv_eps) * slow;
-    } else {
-        const double wr = 1. - v.y * inv_eps, wi = v.x * inv_eps;
-        const double s2 = 2. * slow / (wr * wr + wi * wi);
-        return mk(wr * s2, -wi * s2);
-    }
-}
-
-template <int PRE>
-__device__ __forceinline__ c128 update(c128 dpsi, c128 t, c128 v, double slow, double eps,
-                                       double inv_eps)
-{
-    if constexpr (PRE == PRE_NAIVE) {
-        return t;
-    } else if constexpr (PRE == PRE_IDENTITY) {
-        return slow == 1. ? t : dpsi * (1 - slow) + t * slow;
-    } else {
-        c128 g = gamma_fused<PRE>(v, slow, eps, inv_eps);
-        return mk(1. - g.x, -g.y) * dpsi + g * t;
-    }
-}
 
 // 1/d for normal, finite d: the v_rcp_f64 estimate, then two Newton steps
 // x <- x + x (1 - d x), each of which squares the relative error, so the
@@ -128,13 +56,6 @@ __device__ __forceinline__ c128 mul_g0(c128 a, double wr, double wi)
 {
     const double inv = recip_nr(wr * wr + wi * wi);
     return mk((a.x * wr + a.y * wi) * inv, (a.y * wr - a.x * wi) * inv);
-}
-
-template <int PRE>
-__device__ __forceinline__ c128 source(c128 dpsi, c128 p0, c128 v, double eps)
-{
-    if constexpr (PRE == PRE_NAIVE) return (dpsi + p0) * v;          // op_AddMul
-    else return mk(v.x, v.y + eps) * dpsi + v.x * p0;                // op_Add3
 }
 
 // Launch variant of the Born sweeps per line length (LineV: 8 elements per
@@ -606,7 +527,11 @@ struct qsim_born_job {
     bool plane = false;
     c64 *Vf = nullptr;
     const void *tw[3] = {nullptr, nullptr, nullptr};
-    // unfused path (FP64, any size)
+    // mixed-radix lines (FP64): the fused passes on lengths that are not a
+    // power of two; one plan per axis
+    bool mix = false;
+    MixPlan plan[3]{};
+    // unfused path (FP64, any other size)
     qsim_fft_plan *fwd = nullptr, *inv = nullptr;
     c128 *psi0 = nullptr, *veff = nullptr, *last = nullptr;
 };
@@ -881,6 +806,14 @@ int create(qsim_born_job *j)
     j->prec = d.precision;
     j->fused = born_len_ok(g.n0, j->prec) && born_len_ok(g.ninner, j->prec) &&
                (dim == 2 || born_len_ok(g.n1, j->prec));
+    if (!j->fused && j->prec == 64) {
+        const size_t n[3] = {g.n0, g.n1, g.n2};
+        // radices by the grid alone: an energy's iterates are the same bits
+        // alone and among others
+        j->mix = true;
+        for (int a = 0; a < dim; ++a)
+            j->mix = j->mix && mix_plan(n[a], mix_work(n[a], j->n / n[a]), &j->plan[a]);
+    }
     if (!j->fused && j->prec != 64)
         return set_error(QSIM_ERR_UNSUPPORTED,
                          "FP32 Born job needs power-of-two axes (64..4096)");
@@ -897,7 +830,10 @@ int create(qsim_born_job *j)
     j->resid.assign(j->nE, 0.0);
     j->plane = j->fused && j->prec == 32 && dim == 3 && g.n1 == (size_t)PLANE_N &&
                g.n2 == (size_t)PLANE_N;
-    j->inner_blocks = j->plane ? g.n0 : (j->fused ? inner_blocks(j->prec, g) : 0);
+    j->inner_blocks = j->plane ? g.n0
+                      : j->fused ? inner_blocks(j->prec, g)
+                      : j->mix   ? mix_born_blocks(j->plan[dim - 1], g)
+                                 : 0;
     for (int e = 0; e < j->nE; ++e) {
         BornDev &J = j->host[e];
         const double En = j->E[e];
@@ -952,7 +888,7 @@ int create(qsim_born_job *j)
         QSIM_HIP(hipMemset(p, 0, j->n * esz));
         QSIM_TRY(balloc(j, &p, j->n * esz));
         J.tmp = p;
-        size_t nb = j->fused ? j->inner_blocks : 1;
+        size_t nb = j->fused ? j->inner_blocks : j->mix ? 2 * j->inner_blocks : 1;
         QSIM_TRY(balloc(j, &p, 2 * nb * sizeof(double)));
         J.resid = (double *)p;
     }
@@ -975,7 +911,7 @@ int create(qsim_born_job *j)
     j->rtot_dev = (double *)p;
     QSIM_HIP(hipHostMalloc(&p, 2 * sizeof(double) * j->nE, hipHostMallocDefault));
     j->rtot_host = (double *)p;
-    if (j->fused) {
+    if (j->fused || j->mix) {
         QSIM_TRY(twiddle_table(g.n0, j->prec, &j->tw[0]));
         QSIM_TRY(twiddle_table(g.n1, j->prec, &j->tw[1]));
         if (dim == 3) QSIM_TRY(twiddle_table(g.n2, j->prec, &j->tw[2]));
@@ -1001,6 +937,16 @@ int fused_pass_set(qsim_born_job *j, int mode, const BornDev *tab, int nact, hip
     // mode: BA_START or BA_BOTH starts an iteration and runs it up to the
     // point where only the inner inverse + update remains
     const void *tw_in = j->geo.dim == 3 ? j->tw[2] : j->tw[1];
+    if (j->mix) {
+        QSIM_TRY(mix_born_inner(mode, j->pre, tab, nact, j->V, j->geo, j->plan[j->geo.dim - 1],
+                                tw_in, s));
+        if (j->geo.dim == 3)
+            QSIM_TRY(mix_born_mid(false, tab, nact, j->geo, j->plan[1], j->tw[1], s));
+        QSIM_TRY(mix_born_outer(tab, nact, j->geo, j->plan[0], j->tw[0], s));
+        if (j->geo.dim == 3)
+            QSIM_TRY(mix_born_mid(true, tab, nact, j->geo, j->plan[1], j->tw[1], s));
+        return QSIM_OK;
+    }
     if (j->plane) {
         QSIM_TRY(plane(mode, j->pre, tab, nact, j->Vf, j->geo, tw_in, s));
         return outer(j->prec, tab, nact, j->geo, j->tw[0], s);
@@ -1038,9 +984,13 @@ int read_residuals(qsim_born_job *j, const std::vector<int> &act, hipStream_t s,
     const int nact = (int)act.size();
     out.assign(act.size(), 0.0);
     if (nact == 0) return QSIM_OK;
-    hipLaunchKernelGGL(k_resid_total, dim3((nact + 63) / 64), dim3(64), 0, s,
-                       (const BornDev *)j->active_tab, nact, j->inner_blocks, j->rtot_dev);
-    QSIM_HIP(hipGetLastError());
+    if (j->mix) {
+        QSIM_TRY(mix_born_resid(j->active_tab, nact, j->inner_blocks, j->rtot_dev, s));
+    } else {
+        hipLaunchKernelGGL(k_resid_total, dim3((nact + 63) / 64), dim3(64), 0, s,
+                           (const BornDev *)j->active_tab, nact, j->inner_blocks, j->rtot_dev);
+        QSIM_HIP(hipGetLastError());
+    }
     QSIM_HIP(hipMemcpyAsync(j->rtot_host, j->rtot_dev, 2 * sizeof(double) * nact,
                             hipMemcpyDeviceToHost, s));
     QSIM_HIP(hipStreamSynchronize(s));
@@ -1056,7 +1006,9 @@ int fused_iterate(qsim_born_job *j, int max_iter, double tol, hipStream_t s)
     std::vector<int> act;
     for (int e = 0; e < j->nE; ++e) act.push_back(e);
     std::vector<int> done_it(j->nE, 0);
-    const int check_every = tol > 0 ? 4 : 0;
+    // mixed-radix grids stop at the first update below the tolerance, as the
+    // unfused order does
+    const int check_every = tol > 0 ? (j->mix ? 1 : 4) : 0;
     int it = 0;
     auto upload_tab = [&]() -> int {
         // the previous upload has completed (each one ends with a stream sync)
@@ -1101,7 +1053,11 @@ int fused_iterate(qsim_born_job *j, int max_iter, double tol, hipStream_t s)
     }
     if (!act.empty()) {
         // finish the started iteration of every still-active energy
-        if (j->plane)
+        if (j->mix)
+            QSIM_TRY(mix_born_inner(BA_END, j->pre, j->active_tab, (int)act.size(), j->V, j->geo,
+                                    j->plan[j->geo.dim - 1],
+                                    j->geo.dim == 3 ? j->tw[2] : j->tw[1], s));
+        else if (j->plane)
             QSIM_TRY(plane(BA_END, j->pre, j->active_tab, (int)act.size(), j->Vf, j->geo,
                            j->tw[2], s));
         else
@@ -1232,7 +1188,7 @@ int qsim_hip_born_iterate(qsim_born_job *j, int max_iter, double tol, int *iters
     hipStream_t s = as_stream(stream);
     for (int e = 0; e < j->nE; ++e) j->iters[e] = 0;
     if (max_iter > 0) {
-        if (j->fused) QSIM_TRY(fused_iterate(j, max_iter, tol, s));
+        if (j->fused || j->mix) QSIM_TRY(fused_iterate(j, max_iter, tol, s));
         else QSIM_TRY(unfused_iterate(j, max_iter, tol, s));
     }
     QSIM_HIP(hipStreamSynchronize(s));

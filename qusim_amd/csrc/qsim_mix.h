@@ -427,11 +427,14 @@ __device__ __forceinline__ MixWg<T> mix_begin(unsigned char *smem, const MixPlan
     return MixWg<T>{lds, lds + d.alt, t, (int)threadIdx.x, d.nt, d.logl, d.sh};
 }
 
-// The four kinds of pass.  FIRST reads `in` and has no twiddles; LAST writes
-// `out`; TURN is the last pass of one transform, the pointwise stage `mid`
+// vmcnt(0): the table's loads are done (before a barrier)
+__device__ __forceinline__ void mix_wait_table() { __builtin_amdgcn_s_waitcnt(0x0f70); }
+
+// The kinds of pass.  FIRST reads `in` and has no twiddles; HEAD is a first
+// pass on lines that are in LDS already; LAST writes `out`; TURN is the last pass of one transform, the pointwise stage `mid`
 // and the first pass of the next transform (whose first radix is this one's
 // last, so its inputs are already in the right registers).
-enum { MIX_FIRST = 0, MIX_MID = 1, MIX_TURN = 2, MIX_LAST = 3 };
+enum { MIX_FIRST = 0, MIX_MID = 1, MIX_TURN = 2, MIX_LAST = 3, MIX_HEAD = 4 };
 
 // pre(l, m): the factor of `mid` and `out` at element m, loaded at the top of
 // the pass so that it lands while the butterflies run; fn(l, m, v, factor).
@@ -461,7 +464,7 @@ __device__ __forceinline__ void mix_pass_r(const MixWg<T> &w, const MixPass &p, 
                 for (int r = 0; r < R; ++r)
                     f[PRE ? r : 0] = KIND == MIX_LAST ? pre(l, base + r * p.ns) : pre(l, j + r * p.nb);
             }
-            if constexpr (KIND != MIX_FIRST)
+            if constexpr (KIND != MIX_FIRST && KIND != MIX_HEAD)
                 if (u == 0) tw.load(w.tw, mix_mod(p, j) * p.tws);
 #pragma unroll
             for (int r = 0; r < R; ++r)
@@ -470,7 +473,7 @@ __device__ __forceinline__ void mix_pass_r(const MixWg<T> &w, const MixPass &p, 
         }
     }
     // in place: everything read before anything is overwritten
-    if constexpr (KIND == MIX_MID || KIND == MIX_TURN)
+    if constexpr (KIND == MIX_MID || KIND == MIX_TURN || KIND == MIX_HEAD)
         if (w.lds == w.alt) __syncthreads();
 #pragma unroll
     for (int u = 0; u < K; ++u) {
@@ -478,7 +481,7 @@ __device__ __forceinline__ void mix_pass_r(const MixWg<T> &w, const MixPass &p, 
         if (q < total) {
             const int l = q & lm, j = q >> w.logl;
             const int k = KIND == MIX_TURN ? j : mix_mod(p, j), base = (j - k) * R + k;
-            if constexpr (KIND != MIX_FIRST) {
+            if constexpr (KIND != MIX_FIRST && KIND != MIX_HEAD) {
                 if (u > 0) tw.load(w.tw, k * p.tws);
                 tw.dft(v[u]);
             } else {
@@ -504,7 +507,7 @@ __device__ __forceinline__ void mix_pass_r(const MixWg<T> &w, const MixPass &p, 
             }
         }
     }
-    if constexpr (KIND == MIX_FIRST) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the table
+    if constexpr (KIND == MIX_FIRST) mix_wait_table();
     if constexpr (KIND != MIX_LAST) __syncthreads();
 }
 

@@ -70,3 +70,51 @@ def test_2d_mixed_radix_matches_oracle(shape, method, oracle):
     ref = oracle.split2d(psi, V, L0[0], L0[1], L1[0], L1[1], 0.05, 6, method=method,
                          complex_v=True)
     assert rel_l2(got, ref) < 1e-12
+
+
+def _born(shape, E, pre, precision="fp64", order=5):
+    from test_gpu_born import opts, pot2d, pot3d
+    from qusim_amd.api import QuPerturbation2D, QuPerturbation3D, SolverMethod
+    lo = tuple(-s / 2.0 for s in shape)
+    hi = tuple(s / 2.0 for s in shape)
+    d = (0.3, -0.5, 0.8)[:len(shape)]
+    box = [v for s, a, b in zip(shape, lo, hi) for v in (a, b, s)]
+    V = (pot2d if len(shape) == 2 else pot3d)(shape, lo, hi)
+    cls = QuPerturbation2D if len(shape) == 2 else QuPerturbation3D
+    s = cls().init(V, *box, E, 0.01, *d, SolverMethod.BornSerise, 1.0, 1.0,
+                   opts(pre != 4, min(pre, 3), 0.7, order, precision=precision))
+    return s, V, lo, hi, d
+
+
+# shortest axes, one that needs several radices, a power of two among them, a
+# plane that the last workgroup does not fill; every preconditioner (4: none)
+@pytest.mark.parametrize("shape", [(4, 300), (300, 6), (250, 350), (4, 6, 250), (26, 64, 33),
+                                   (32, 32, 32)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("pre", [0, 1, 2, 3, 4])
+def test_born_mixed_radix_matches_oracle(shape, pre, oracle):
+    if pre != 4 and min(shape) < 20:
+        pytest.skip("the preconditioned solver refuses boxes this small")
+    E = 6.0 if len(shape) == 2 else 2.0
+    if len(shape) == 2 and pre != 4:
+        E = (1.1 * 24 * 2 * np.pi / min(shape)) ** 2 / 2
+    s, V, lo, hi, d = _born(shape, E, pre)
+    s.Compute()
+    ref, _, _, _ = oracle.born(V, lo, hi, E, d, order=5, preconditional=int(pre != 4),
+                               preconditioner=min(pre, 3), slow=0.7, epsilon=0.01, threads=8)
+    assert rel_l2(s.GetPsi(), ref) < 1e-12
+
+
+def test_born_mixed_radix_stops_at_the_first_update_below_the_tolerance():
+    shape, E = (24, 20, 28), [2.0, 2.6]
+    one, _, _, _, _ = _born(shape, E, 1, order=1)
+    res = []
+    for _ in range(7):
+        one.Compute()
+        res.append(list(one.residual))
+    many, _, _, _, _ = _born(shape, E, 1)
+    tol = 0.5 * (res[3][0] + res[4][0])
+    many.Compute(max_iter=7, tol=tol)
+    want = [next((k + 1 for k in range(7) if res[k][e] < tol), 7) for e in range(2)]
+    assert many.iters == want and want[0] == 5
+    for e in range(2):
+        assert abs(many.residual[e] / res[want[e] - 1][e] - 1) < 1e-13

@@ -44,6 +44,7 @@ struct MixPass {
 struct MixPlan {
     int n, nf;
     int tlen;                       // table entries that the passes use
+    int prime;                      // has passes of a prime above 13
     MixPass f[2 * kMixMaxPasses];   // radices r0, r1, ... of the first transform;
                                     // from kMixMaxPasses on, in reverse order
 };
@@ -53,7 +54,7 @@ struct MixPlan {
 // registers of a 1024-thread workgroup.
 __host__ __device__ constexpr int mix_k(int R)
 {
-    return R == 2 ? 4 : R == 3 ? 3 : R <= 7 ? 2 : 1;
+    return R == 1 ? 8 : R == 2 ? 4 : R == 3 ? 3 : R <= 7 ? 2 : 1;
 }
 
 // Slot of LDS element e: one element of padding per 8 (sh = 3), or per 16
@@ -164,6 +165,13 @@ template <> struct MixDft<7> : MixPrime<7> {};
 template <> struct MixDft<11> : MixPrime<11> {};
 template <> struct MixDft<13> : MixPrime<13> {};
 
+// A first or last pass that only loads or stores, beside a prime's pass.
+template <>
+struct MixDft<1> {
+    static constexpr int PAIRS = 0;
+    static __host__ __device__ constexpr int pair(int, int) { return 0; }
+    static __host__ __device__ __forceinline__ void rest(c128 *) {}
+};
 template <>
 struct MixDft<2> {
     static constexpr int PAIRS = 1;
@@ -511,6 +519,66 @@ __device__ __forceinline__ void mix_pass_r(const MixWg<T> &w, const MixPass &p, 
     if constexpr (KIND != MIX_LAST) __syncthreads();
 }
 
+// A pass of a prime P above 13.  First the twiddled inputs' pairs (k, P - k),
+// in place: a_k = x_k + x_{P-k}, b_k = x_k - x_{P-k}; then the outputs m and
+// P - m of butterfly j, X = x_0 + sum_k a_k cos(2 pi k m / P) -+ i sum_k b_k
+// sin(2 pi k m / P).  at(e): element e of the line.  Against one sum of P
+// terms per output it takes half the LDS reads, and its error is smaller.
+template <typename At>
+__host__ __device__ __forceinline__ void mix_prime_pair(const MixPass &p, const c128 *tw, int j,
+                                                        int k, At at)
+{
+    const int e = k * mix_mod(p, j) * p.tws, f = (p.R - k) * mix_mod(p, j) * p.tws;
+    const c128 x = at.get(j + k * p.nb) * tw[e], y = at.get(j + (p.R - k) * p.nb), w = tw[f];
+    at.set(j + k * p.nb, mix_fma(x, y, w));
+    at.set(j + (p.R - k) * p.nb, mix_fms(x, y, w));
+}
+template <typename At, typename Out>
+__host__ __device__ __forceinline__ void mix_prime_out(const MixPass &p, const c128 *tw, int j,
+                                                       int m, At at, Out out)
+{
+    const int P = p.R, k0 = mix_mod(p, j), base = (j - k0) * P + k0;
+    c128 e = at.get(j), o = mk(0.0, 0.0);
+    int q = 0;
+    for (int k = 1; 2 * k < P; ++k) {
+        q += m;
+        if (q >= P) q -= P;
+        const c128 w = tw[q * p.nb], a = at.get(j + k * p.nb), b = at.get(j + (P - k) * p.nb);
+        e = mk(fma(w.x, a.x, e.x), fma(w.x, a.y, e.y));
+        o = mk(fma(-w.y, b.y, o.x), fma(w.y, b.x, o.y));   // i sum w.y b
+    }
+    out(base + m * p.ns, e + o);
+    if (m > 0) out(base + (P - m) * p.ns, e - o);
+}
+
+template <typename T>
+__device__ __forceinline__ void mix_prime(const MixWg<T> &w, const MixPass &p)
+{
+    struct At {
+        const MixWg<T> &w;
+        int l;
+        __device__ __forceinline__ c128 get(int e) const { return mix_ld(w, l, e); }
+        __device__ __forceinline__ void set(int e, c128 v) const
+        {
+            w.lds[mix_slot((e << w.logl) + l, w.sh)] = cvt<T>(v);
+        }
+    };
+    const int lm = (1 << w.logl) - 1, H = (p.R - 1) / 2;
+    const unsigned mag = p.nb == 1 ? 0u : 0xffffffffu / (unsigned)p.nb + 1u;
+    const int pairs = (p.nb * H) << w.logl, outs = (p.nb * (H + 1)) << w.logl;
+    for (int q = w.tid; q < pairs; q += w.nt) {
+        const int t = q >> w.logl, k = p.nb == 1 ? t : (int)mix_mulhi((unsigned)t, mag);
+        mix_prime_pair(p, w.tw, t - k * p.nb, k + 1, At{w, q & lm});
+    }
+    __syncthreads();
+    for (int q = w.tid; q < outs; q += w.nt) {
+        const int t = q >> w.logl, m = p.nb == 1 ? t : (int)mix_mulhi((unsigned)t, mag);
+        mix_prime_out(p, w.tw, t - m * p.nb, m, At{w, q & lm},
+                      [&](int e, c128 v) { mix_st(w, q & lm, e, v); });
+    }
+    __syncthreads();
+}
+
 template <int KIND, int PREMAX = 9, typename T, typename Pre, typename F>
 __device__ __forceinline__ void mix_pass(MixWg<T> &w, const MixPass &pass, Pre pre, F fn)
 {
@@ -524,11 +592,13 @@ __device__ __forceinline__ void mix_pass(MixWg<T> &w, const MixPass &pass, Pre p
     switch (p.R) {
 #define QSIM_MIX_R(R_) \
     case R_: mix_pass_r<KIND, R_, PREMAX>(wq, p, pre, fn); break;
-        QSIM_MIX_R(2) QSIM_MIX_R(3) QSIM_MIX_R(4) QSIM_MIX_R(5) QSIM_MIX_R(6) QSIM_MIX_R(7)
+        QSIM_MIX_R(1) QSIM_MIX_R(2) QSIM_MIX_R(3) QSIM_MIX_R(4) QSIM_MIX_R(5) QSIM_MIX_R(6) QSIM_MIX_R(7)
         QSIM_MIX_R(8) QSIM_MIX_R(9) QSIM_MIX_R(10) QSIM_MIX_R(11) QSIM_MIX_R(12) QSIM_MIX_R(13)
         QSIM_MIX_R(14) QSIM_MIX_R(15)
 #undef QSIM_MIX_R
-        default: break;
+        default:
+            if constexpr (KIND == MIX_MID) mix_prime(wq, p);
+            break;
     }
     if constexpr (KIND != MIX_LAST) {
         w.lds = wq.alt;
@@ -610,14 +680,40 @@ inline void mix_split(int n, int maxr, int depth, double work, double cost, int 
 }
 
 // `work`: line elements that a CU holds at a time.  false when n is not a
-// composite number with prime factors of at most 13, 4 <= n <= kMixMaxLen.
+// composite number with prime factors of at most 13, 4 <= n <= kMixMaxLen, or
+// any number with a larger prime factor whose line fits LDS twice (mix_fits:
+// up to 3150 points).
+bool mix_fits(const MixPlan &p);
 inline bool mix_plan(size_t n, double work, MixPlan *p)
 {
     if (n < 4 || n > (size_t)kMixMaxLen) return false;
+    int primes[kMixMaxPasses], np = 0, s = (int)n;
+    for (int q = 17; q <= s; q += 2)
+        while (s % q == 0) {   // q is prime or s has lost its factors
+            bool is_prime = true;
+            for (int d = 3; d * d <= q; d += 2) is_prime = is_prime && q % d;
+            if (!is_prime) break;
+            if (np == kMixMaxPasses - 2) return false;
+            primes[np++] = q;
+            s /= q;
+        }
     int cur[kMixMaxPasses], best[kMixMaxPasses], nf = 0;
     double cost = 1e300;
-    mix_split((int)n, 15, 0, work, 0, cur, best, &nf, &cost);
+    if (s > 1) mix_split(s, 15, 0, work, 0, cur, best, &nf, &cost);
+    if (np > 0) {
+        // the primes in the middle, between radices that may be 1
+        if (nf == 0 && s <= 15) {
+            best[0] = s;
+            best[1] = 1;
+            nf = 2;
+        }
+        if (nf == 0 || nf + np > kMixMaxPasses) return false;
+        for (int i = nf - 1; i >= 1; --i) best[i + np] = best[i];
+        for (int i = 0; i < np; ++i) best[1 + i] = primes[i];
+        nf += np;
+    }
     if (nf == 0) return false;
+    p->prime = np > 0;
     p->n = (int)n;
     p->nf = nf;
     p->tlen = 0;
@@ -631,12 +727,13 @@ inline bool mix_plan(size_t n, double work, MixPlan *p)
             f[i].ns = ns;
             f[i].mag = ns == 1 ? 0u : (unsigned)((0x100000000ull + ns - 1) / ns);
             f[i].tws = (int)n / (ns * R);
-            const int top = (R - 1) * (ns - 1) * f[i].tws + 1;
+            int top = (R - 1) * (ns - 1) * f[i].tws + 1;
+            if (R > 15 && (R - 1) * f[i].nb >= top) top = (R - 1) * f[i].nb + 1;
             if (top > p->tlen) p->tlen = top;
             ns *= R;
         }
     }
-    return true;
+    return mix_fits(*p);
 }
 
 // Elements of `nlines` lines of n points that one of 256 CUs holds at a time:
@@ -660,7 +757,14 @@ inline int mix_threads(const MixPlan &p, int L)
 {
     int nt = 64;
     for (int i = 0; i < p.nf; ++i) {
-        const int R = p.f[i].R, total = p.f[i].nb * L, per = total <= 512 ? 1 : mix_k(R);
+        const int R = p.f[i].R, total = p.f[i].nb * L;
+        if (R > 15) {   // its outputs are a loop
+            int t = (p.f[i].nb * (R + 1) / 2 * L + 63) / 64 * 64;
+            if (t > 512) t = 512;
+            if (t > nt) nt = t;
+            continue;
+        }
+        const int per = total <= 512 && R > 1 ? 1 : mix_k(R);
         int t = ((total + per - 1) / per + 63) / 64 * 64;
         if (t > kMixMaxThreads) return 0;
         if (t > nt) nt = t;
@@ -684,12 +788,19 @@ inline MixShape mix_shape_of(const MixPlan &p, int lg, size_t nlines, size_t ele
     }
     s.lds = tab + elems * elem_bytes;
     if (s.lds > kMixMaxLds) s.d.nt = 0;
+    // a prime's pass does not run in place
+    if (p.prime) {
+        pair = kMixMaxLds;
+        if (s.lds + elems * elem_bytes > pair) s.d.nt = 0;
+    }
     if (s.lds + elems * elem_bytes <= pair) {
         s.d.alt = (int)elems;
         s.lds += elems * elem_bytes;
     }
     return s;
 }
+
+inline bool mix_fits(const MixPlan &p) { return mix_shape_of(p, 0, 1, sizeof(c128), 0).d.nt > 0; }
 
 inline MixShape mix_shape(const MixPlan &p, size_t nlines, size_t elem_bytes, bool strided)
 {

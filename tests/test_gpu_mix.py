@@ -12,7 +12,10 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(4,), (6,), (9,), (15,), (1000,), (3003,), (5000,), (5103,), (5120,), (4900,),
           (4, 6), (6, 1000), (1000, 6), (100, 169), (143, 77), (1500, 1100), (1, 60), (60, 1),
-          (9, 10, 12), (14, 15, 98), (100, 120, 90), (17, 60, 50)]
+          (9, 10, 12), (14, 15, 98), (100, 120, 90), (17, 60, 50),
+          # a prime above 13 alone, with others, twice, beside one line per workgroup
+          (17,), (34,), (323,), (850,), (1369,), (2003,), (3109,), (3150,), (59, 118), (1009, 20),
+          (23, 38, 62)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -32,7 +35,8 @@ def test_fft_mixed_radix(shape, precision):
     assert rel_l2(fftn(x, inverse=True, precision=precision), np.fft.ifftn(xd) * x.size) < tol
 
 
-@pytest.mark.parametrize("n", [4, 12, 60, 1000, 1300, 3003, 5082, 5103, 5120])
+@pytest.mark.parametrize("n", [4, 12, 60, 1000, 1300, 3003, 5082, 5103, 5120,
+                               17, 850, 1009, 3109])
 @pytest.mark.parametrize("method", [2, 4])
 def test_1d_mixed_radix_matches_oracle(n, method, oracle):
     x = -25.0 + 50.0 / n * np.arange(n)
@@ -48,7 +52,7 @@ def test_1d_mixed_radix_matches_oracle(n, method, oracle):
     assert rel_l2(f.GetPsi(), g) < 1e-12
 
 
-@pytest.mark.parametrize("n", [2, 15, 500, 1024, 1500, 2560])
+@pytest.mark.parametrize("n", [2, 15, 500, 1024, 1500, 2560, 17, 517, 1549])
 @pytest.mark.parametrize("method", [2, 4])
 def test_wall_mixed_radix_matches_oracle(n, method, oracle):
     """the odd extension to 2n points; psi(0) is not zero at the start"""
@@ -61,7 +65,8 @@ def test_wall_mixed_radix_matches_oracle(n, method, oracle):
 
 
 @pytest.mark.parametrize("shape", [(4, 4), (6, 1000), (1000, 6), (65, 130), (750, 600),
-                                   (1024, 250), (98, 2048), (5120, 12), (32, 32)],
+                                   (1024, 250), (98, 2048), (5120, 12), (32, 32),
+                                   (34, 59), (850, 101), (64, 1009), (3109, 17)],
                          ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("method", [2, 4])
 def test_2d_mixed_radix_matches_oracle(shape, method, oracle):
@@ -89,6 +94,7 @@ def _born(shape, E, pre, precision="fp64", order=5):
 # shortest axes, one that needs several radices, a power of two among them, a
 # plane that the last workgroup does not fill; every preconditioner (4: none)
 @pytest.mark.parametrize("shape", [(4, 300), (300, 6), (250, 350), (4, 6, 250), (26, 64, 33),
+                                   (34, 251), (23, 38, 51),
                                    (32, 32, 32)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("pre", [0, 1, 2, 3, 4])
 def test_born_mixed_radix_matches_oracle(shape, pre, oracle):

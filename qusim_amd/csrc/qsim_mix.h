@@ -160,7 +160,26 @@ struct MixPrime {
     }
 };
 template <> struct MixDft<3> : MixPrime<3> {};
-template <> struct MixDft<5> : MixPrime<5> {};
+// 5: the cosines' mean is -1/4 exactly, so the even part takes one rounded
+// constant, sqrt(5) / 4, instead of two.
+template <>
+struct MixDft<5> : MixPrime<5> {
+    static __host__ __device__ __forceinline__ void rest(c128 *v)
+    {
+        constexpr double k = 0.55901699437494742410, s1 = MixC<5>::s[0], s2 = MixC<5>::s[1];
+        const c128 x0 = v[0], a = v[1] + v[2], d = v[1] - v[2], b1 = v[4], b2 = v[3];
+        const c128 t = mk(fma(-0.25, a.x, x0.x), fma(-0.25, a.y, x0.y));
+        const c128 e1 = mk(fma(k, d.x, t.x), fma(k, d.y, t.y));
+        const c128 e2 = mk(fma(-k, d.x, t.x), fma(-k, d.y, t.y));
+        const c128 o1 = mk(fma(s1, b1.y, s2 * b2.y), -fma(s1, b1.x, s2 * b2.x));   // -i o
+        const c128 o2 = mk(fma(s2, b1.y, -(s1 * b2.y)), fma(-s2, b1.x, s1 * b2.x));
+        v[0] = x0 + a;
+        v[1] = e1 + o1;
+        v[4] = e1 - o1;
+        v[2] = e2 + o2;
+        v[3] = e2 - o2;
+    }
+};
 template <> struct MixDft<7> : MixPrime<7> {};
 template <> struct MixDft<11> : MixPrime<11> {};
 template <> struct MixDft<13> : MixPrime<13> {};

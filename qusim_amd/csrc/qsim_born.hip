@@ -118,12 +118,12 @@ static bool stream_nt(size_t bytes_per_launch) { return bytes_per_launch >= ((si
 // (i, j) = (g / nmid, g % nmid) in 3D, i = g in 2D.  The operands of the
 // update (dpsi, V) are loaded before the inverse transform, so their latency
 // hides behind it.
-template <typename T, int N, int MODE, int PRE, bool NT>
-__global__ void __launch_bounds__((P2Launch<T, N, false, BornV<N>::V>::THREADS))
+template <typename T, int N, int MODE, int PRE, bool NT, bool NARROW>
+__global__ void __launch_bounds__((P2Launch<T, N, false, BornV<N>::V, NARROW>::THREADS))
     k_born_inner(const BornDev *__restrict__ jobs, const c128 *__restrict__ V, BornGeom geo,
                  const c128 *__restrict__ tw)
 {
-    using LP = P2Launch<T, N, false, BornV<N>::V>;
+    using LP = P2Launch<T, N, false, BornV<N>::V, NARROW>;
     using P = typename LP::Line;
     constexpr int L = LP::L;
     extern __shared__ unsigned char smem_raw[];
@@ -384,11 +384,11 @@ __global__ void __launch_bounds__(PLANE_THREADS)
 }
 
 // Outer sweep: lines along axis 0, stride S = n1*n2, G0 between FFT and IFFT.
-template <typename T, int N, bool NT>
-__global__ void __launch_bounds__((P2Launch<T, N, true, BornLFV<N>::V>::THREADS))
+template <typename T, int N, bool NT, bool NARROW>
+__global__ void __launch_bounds__((P2Launch<T, N, true, BornLFV<N>::V, NARROW>::THREADS))
     k_born_outer(const BornDev *__restrict__ jobs, BornGeom geo, const c128 *__restrict__ tw)
 {
-    using LP = P2Launch<T, N, true, BornLFV<N>::V>;
+    using LP = P2Launch<T, N, true, BornLFV<N>::V, NARROW>;
     using P = typename LP::Line;
     constexpr int L = LP::L;
     extern __shared__ unsigned char smem_raw[];
@@ -397,7 +397,7 @@ __global__ void __launch_bounds__((P2Launch<T, N, true, BornLFV<N>::V>::THREADS)
     const int tid = threadIdx.x;
     const int l = tid % L, t = tid / L;
     const size_t S = geo.n1 * geo.n2;
-    const size_t cidx = (size_t)blockIdx.x * L + l;
+    const size_t cidx = (NARROW ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x) * L + l;
     const bool active = cidx < S;
     const size_t c = active ? cidx : 0;
     cx<T> *tmp = reinterpret_cast<cx<T> *>(J.tmp);
@@ -515,8 +515,8 @@ struct qsim_born_job {
     BornDev *dev = nullptr;     // device copy of `host`
     BornDev *active_tab = nullptr;
     BornDev *tab_host = nullptr;  // pinned staging of the active table
-    double *rtot_dev = nullptr;   // per active energy: residual and norm totals
-    double *rtot_host = nullptr;  // pinned copy of rtot_dev
+    std::vector<int> tab_act;     // the energies that active_tab holds
+    double *rtot_host = nullptr;  // pinned: residual and norm totals per active energy
     std::vector<void *> owned;
     std::vector<bool> started;  // tmp holds a started iteration
     std::vector<int> iters;
@@ -585,17 +585,18 @@ bool born_len_ok(size_t n, int prec)
     }                                                                                 \
     return set_error(QSIM_ERR_UNSUPPORTED, "no fused Born kernel for this length");
 
-template <typename T, int N, int MODE, int PRE>
-int launch_inner_t(const BornDev *tab, int nact, const c128 *V, const BornGeom &geo,
+template <typename T, int N, int MODE, int PRE, bool NARROW>
+int launch_inner_l(const BornDev *tab, int nact, const c128 *V, const BornGeom &geo,
                    const void *tw, hipStream_t s)
 {
-    using LP = P2Launch<T, N, false, BornV<N>::V>;
+    using LP = P2Launch<T, N, false, BornV<N>::V, NARROW>;
     size_t nlines = geo.n0 * geo.nmid;
     // V is what the hint protects, and only other energies of the same
     // launch re-read it soon: complex128 128^3 x 8 energies 1.54 -> 1.61e4
     // energy-iterations/s, one energy unchanged (-1%) so it keeps plain loads
     const bool nt = nact >= 2 && stream_nt((size_t)nact * nlines * N * sizeof(cx<T>));
-    auto fn = nt ? k_born_inner<T, N, MODE, PRE, true> : k_born_inner<T, N, MODE, PRE, false>;
+    auto fn = nt ? k_born_inner<T, N, MODE, PRE, true, NARROW>
+                 : k_born_inner<T, N, MODE, PRE, false, NARROW>;
     QSIM_TRY(lds_limit((const void *)fn, LP::LDS_BYTES));
     dim3 grid((unsigned)((nlines + LP::L - 1) / LP::L), (unsigned)nact);
     hipLaunchKernelGGL(fn, grid, dim3(LP::THREADS), LP::LDS_BYTES, s, tab, V, geo,
@@ -604,11 +605,31 @@ int launch_inner_t(const BornDev *tab, int nact, const c128 *V, const BornGeom &
     return QSIM_OK;
 }
 
+// The inner sweep's shape follows the grid alone (not the energies), so an
+// energy's residual sums are the same alone and among others.
+template <typename T, int N>
+bool inner_narrow(const BornGeom &geo)
+{
+    using LP = P2Launch<T, N, false, BornV<N>::V>;
+    return N <= 1024 && geo.dim == 2 && narrow_launch((geo.n0 * geo.nmid + LP::L - 1) / LP::L);
+}
+
+template <typename T, int N, int MODE, int PRE>
+int launch_inner_t(const BornDev *tab, int nact, const c128 *V, const BornGeom &geo,
+                   const void *tw, hipStream_t s)
+{
+    if constexpr (N <= 1024)
+        if (inner_narrow<T, N>(geo))
+            return launch_inner_l<T, N, MODE, PRE, true>(tab, nact, V, geo, tw, s);
+    return launch_inner_l<T, N, MODE, PRE, false>(tab, nact, V, geo, tw, s);
+}
+
 template <typename T, int N>
 size_t inner_blocks_t(const BornGeom &geo)
 {
-    using LP = P2Launch<T, N, false, BornV<N>::V>;
-    return (geo.n0 * geo.nmid + LP::L - 1) / LP::L;
+    const size_t L = inner_narrow<T, N>(geo) ? P2Launch<T, N, false, BornV<N>::V, true>::L
+                                             : P2Launch<T, N, false, BornV<N>::V>::L;
+    return (geo.n0 * geo.nmid + L - 1) / L;
 }
 
 template <typename T, int N, int MODE>
@@ -692,19 +713,30 @@ size_t inner_blocks(int prec, const BornGeom &geo)
 #undef IB
 }
 
-template <typename T, int N>
-int launch_outer_t(const BornDev *tab, int nact, const BornGeom &geo, const void *tw,
+template <typename T, int N, bool NARROW>
+int launch_outer_l(const BornDev *tab, int nact, const BornGeom &geo, const void *tw,
                    hipStream_t s)
 {
-    using LP = P2Launch<T, N, true, BornLFV<N>::V>;
+    using LP = P2Launch<T, N, true, BornLFV<N>::V, NARROW>;
     size_t S = geo.n1 * geo.n2;
-    auto fn = stream_nt((size_t)nact * S * N * sizeof(cx<T>)) ? k_born_outer<T, N, true>
-                                                               : k_born_outer<T, N, false>;
+    auto fn = stream_nt((size_t)nact * S * N * sizeof(cx<T>)) ? k_born_outer<T, N, true, NARROW>
+                                                               : k_born_outer<T, N, false, NARROW>;
     QSIM_TRY(lds_limit((const void *)fn, LP::LDS_BYTES));
     dim3 grid((unsigned)((S + LP::L - 1) / LP::L), (unsigned)nact);
     hipLaunchKernelGGL(fn, grid, dim3(LP::THREADS), LP::LDS_BYTES, s, tab, geo, (const c128 *)tw);
     QSIM_HIP(hipGetLastError());
     return QSIM_OK;
+}
+
+template <typename T, int N>
+int launch_outer_t(const BornDev *tab, int nact, const BornGeom &geo, const void *tw,
+                   hipStream_t s)
+{
+    using LP = P2Launch<T, N, true, BornLFV<N>::V>;
+    if constexpr (N <= 1024)
+        if (narrow_launch((geo.n1 * geo.n2 + LP::L - 1) / LP::L * nact))
+            return launch_outer_l<T, N, true>(tab, nact, geo, tw, s);
+    return launch_outer_l<T, N, false>(tab, nact, geo, tw, s);
 }
 
 int outer(int prec, const BornDev *tab, int nact, const BornGeom &geo, const void *tw,
@@ -907,8 +939,6 @@ int create(qsim_born_job *j)
     j->active_tab = (BornDev *)p;
     QSIM_HIP(hipHostMalloc(&p, sizeof(BornDev) * j->nE, hipHostMallocDefault));
     j->tab_host = (BornDev *)p;
-    QSIM_TRY(balloc(j, &p, 2 * sizeof(double) * j->nE));
-    j->rtot_dev = (double *)p;
     QSIM_HIP(hipHostMalloc(&p, 2 * sizeof(double) * j->nE, hipHostMallocDefault));
     j->rtot_host = (double *)p;
     if (j->fused || j->mix) {
@@ -958,26 +988,37 @@ int fused_pass_set(qsim_born_job *j, int mode, const BornDev *tab, int nact, hip
     return QSIM_OK;
 }
 
-// Totals of the per-block residual sums of each active energy (tab order),
-// one thread per energy adding the blocks in block order.
-__global__ void k_resid_total(const BornDev *__restrict__ tab, int nact, size_t nb,
-                              double *__restrict__ out)
+// Totals of the per-block residual sums of each active energy (tab order): one
+// workgroup per energy brings the sums to LDS, one thread adds them in block
+// order.  (One thread reading them from memory took 13 us for 128 blocks.)
+constexpr int kResidChunk = 1024;
+__global__ void __launch_bounds__(256)
+    k_resid_total(const BornDev *__restrict__ tab, size_t nb, double *__restrict__ out)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= nact) return;
-    const double *p = tab[a].resid;
+    __shared__ double sh[2 * kResidChunk];
+    const double *p = tab[blockIdx.x].resid;
     double r = 0, nn = 0;
-    for (size_t b = 0; b < nb; ++b) {
-        r += p[2 * b];
-        nn += p[2 * b + 1];
+    for (size_t b0 = 0; b0 < nb; b0 += kResidChunk) {
+        const int m = (int)(nb - b0 < kResidChunk ? nb - b0 : kResidChunk);
+        __syncthreads();
+        for (int i = threadIdx.x; i < 2 * m; i += 256) sh[i] = p[2 * b0 + i];
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int i = 0; i < m; ++i) {
+                r += sh[2 * i];
+                nn += sh[2 * i + 1];
+            }
     }
-    out[2 * a] = r;
-    out[2 * a + 1] = nn;
+    if (threadIdx.x == 0) {
+        out[2 * blockIdx.x] = r;
+        out[2 * blockIdx.x + 1] = nn;
+    }
 }
 
 // Relative update of each active energy, sqrt(sum |d new - d old|^2 /
 // sum |d new|^2); `act` lists the energies of the device's active table in
-// its order.  One small kernel and one copy, then a wait on the stream.
+// its order.  One small kernel that writes to pinned host memory, then a wait
+// on the stream.
 int read_residuals(qsim_born_job *j, const std::vector<int> &act, hipStream_t s,
                    std::vector<double> &out)
 {
@@ -985,14 +1026,12 @@ int read_residuals(qsim_born_job *j, const std::vector<int> &act, hipStream_t s,
     out.assign(act.size(), 0.0);
     if (nact == 0) return QSIM_OK;
     if (j->mix) {
-        QSIM_TRY(mix_born_resid(j->active_tab, nact, j->inner_blocks, j->rtot_dev, s));
+        QSIM_TRY(mix_born_resid(j->active_tab, nact, j->inner_blocks, j->rtot_host, s));
     } else {
-        hipLaunchKernelGGL(k_resid_total, dim3((nact + 63) / 64), dim3(64), 0, s,
-                           (const BornDev *)j->active_tab, nact, j->inner_blocks, j->rtot_dev);
+        hipLaunchKernelGGL(k_resid_total, dim3(nact), dim3(256), 0, s,
+                           (const BornDev *)j->active_tab, j->inner_blocks, j->rtot_host);
         QSIM_HIP(hipGetLastError());
     }
-    QSIM_HIP(hipMemcpyAsync(j->rtot_host, j->rtot_dev, 2 * sizeof(double) * nact,
-                            hipMemcpyDeviceToHost, s));
     QSIM_HIP(hipStreamSynchronize(s));
     for (int a = 0; a < nact; ++a) {
         const double r = j->rtot_host[2 * a], nn = j->rtot_host[2 * a + 1];
@@ -1011,11 +1050,16 @@ int fused_iterate(qsim_born_job *j, int max_iter, double tol, hipStream_t s)
     const int check_every = tol > 0 ? (j->mix ? 1 : 4) : 0;
     int it = 0;
     auto upload_tab = [&]() -> int {
+        // the job's descriptors do not change, so a table of the same energies
+        // is still right (a solve continued by another call)
+        if (j->tab_act == act) return QSIM_OK;
+        j->tab_act.clear();
         // the previous upload has completed (each one ends with a stream sync)
         for (size_t a = 0; a < act.size(); ++a) j->tab_host[a] = j->host[act[a]];
         QSIM_HIP(hipMemcpyAsync(j->active_tab, j->tab_host, sizeof(BornDev) * act.size(),
                                 hipMemcpyHostToDevice, s));
         QSIM_HIP(hipStreamSynchronize(s));
+        j->tab_act = act;
         return QSIM_OK;
     };
     QSIM_TRY(upload_tab());

@@ -91,7 +91,13 @@ __host__ __device__ constexpr int pow2floor(int x) { return x <= 1 ? 1 : 2 * pow
 // Lines per workgroup: rows (position-fast) fill ~256 threads; strided axes
 // (line-fast) take 128 B of adjacent lines per row of the tile; both kept
 // within 96 KiB of LDS and a power of two, unless the variant fixes them.
-template <typename T, int N, bool LF, int V = 0>
+// NARROW: the shape of launches whose ordinary tiles would leave CUs idle
+// (narrow_launch): workgroups of one wave, strided lines at least 32 B of
+// adjacent lines (half a wave of 128-point columns lost: 128 x 1024 FP64 11.9
+// -> 13.3 us a step).  256^2 FP64 10.8 -> 8.9 us a step, 512^2 FP64 15.7 ->
+// 13.2, 512^2 FP32 13.0 -> 10.9, a 2D Born iteration of 512^2 FP32 19.3 ->
+// 16.4.
+template <typename T, int N, bool LF, int V = 0, bool NARROW = false>
 struct P2Launch {
     using Cfg = P2Cfg<T, N, V>;
     using Base = typename Cfg::Line;
@@ -110,7 +116,8 @@ struct P2Launch {
     static constexpr int L_WANT = LF ? LF_LINES : ROWS;
     static constexpr int LS_MAX = Sized::LS_RAW + 15;
     static constexpr int L_LDS = cmax(1, (96 * 1024) / (LS_MAX * (int)sizeof(cx<T>)));
-    static constexpr int L_FIXED = LF ? Cfg::COL_L : Cfg::ROW_L;
+    static constexpr int L_FIXED = NARROW ? cmax(LF ? 32 / (int)sizeof(cx<T>) : 1, 64 / Sized::TPL)
+                                          : (LF ? Cfg::COL_L : Cfg::ROW_L);
     // never more lines than the 160 KiB of LDS one workgroup can hold
     static constexpr int L_CAP = pow2floor(cmax(1, (160 * 1024) / (LS_MAX * (int)sizeof(cx<T>))));
     static constexpr int L = cmin(L_CAP, L_FIXED > 0 ? L_FIXED : pow2floor(cmin(L_WANT, L_LDS)));
@@ -133,6 +140,11 @@ struct P2Launch {
         Line::LS_RAW + (((TARGET - Line::LS_RAW % 16) % 16) + 16) % 16;
     static constexpr size_t LDS_BYTES = (size_t)L * LSTR * sizeof(cx<T>);
 };
+
+// A launch whose ordinary tiles would leave 3 of 8 CUs (of 256) without one
+// takes the narrow shape; at 192 tiles (3 grids of 512^2 FP32) the two measured
+// the same within 5% either way.
+inline bool narrow_launch(size_t blocks) { return blocks < 160; }
 
 // Radix plan of the Born sweeps per length: 8 elements per thread from 128
 // to 4096 points, so a solve of one energy on a few hundred lines still puts

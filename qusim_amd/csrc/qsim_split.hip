@@ -487,12 +487,12 @@ __global__ void __launch_bounds__((XRowLaunch<T, N, V, R>::THREADS))
             jobs[blockIdx.y], blockIdx.x, nx, iev, tw, twx, reinterpret_cast<cx<T> *>(smem_raw));
 }
 
-template <typename T, int N, int MODE, int V, bool NT>
-__global__ void __launch_bounds__((P2Launch<T, N, false, V>::THREADS))
+template <typename T, int N, int MODE, int V, bool NT, bool NARROW = false>
+__global__ void __launch_bounds__((P2Launch<T, N, false, V, NARROW>::THREADS))
     k_row_sweep(const SplitDev *__restrict__ jobs, size_t nrows, int iev,
                 const c128 *__restrict__ tw)
 {
-    using LP = P2Launch<T, N, false, V>;
+    using LP = P2Launch<T, N, false, V, NARROW>;
     extern __shared__ unsigned char smem_raw[];
     row_lines<T, typename LP::Line, LP::L, LP::LSTR, MODE, NT>(
         jobs[blockIdx.y], (size_t)blockIdx.x * LP::L, nrows, iev, tw,
@@ -559,12 +559,12 @@ __device__ __forceinline__ void col_lines(const SplitDev &J, size_t g0, size_t n
     }
 }
 
-template <typename T, int N, int V, bool NT, int R = 1>
-__global__ void __launch_bounds__((P2Launch<T, N, true, V>::THREADS))
+template <typename T, int N, int V, bool NT, int R = 1, bool NARROW = false>
+__global__ void __launch_bounds__((P2Launch<T, N, true, V, NARROW>::THREADS))
     k_col_sweep(const SplitDev *__restrict__ jobs, size_t ncols, int ik,
                 const c128 *__restrict__ tw)
 {
-    using LP = P2Launch<T, N, true, V>;
+    using LP = P2Launch<T, N, true, V, NARROW>;
     extern __shared__ unsigned char smem_raw[];
     col_lines<T, typename LP::Line, LP::L, LP::LSTR, NT, R>(
         jobs[blockIdx.y], xcd_tile(blockIdx.x, gridDim.x) * LP::L, ncols, ik, tw,
@@ -811,11 +811,46 @@ int build_axis(qsim_split_job *j, c128 **out, size_t n, cd alpha, double a, doub
     return QSIM_OK;
 }
 
+// Variants a new job starts with: the pairs the autotuner picked most often
+// on MI355X for single and batched jobs of these lengths (row variant by the
+// row length ny, column variant by the column length nx).  Fixed, so jobs that
+// are never tuned (request loops, batches) still take a fast pair and two
+// runs of one job always choose the same radix plans.
+// 128- to 512-point lines take the 8-per-thread plan (variant 1): measured
+// on MI355X per step, single job / 16 batched: 128^2 FP32 11.7 -> 9.6 /
+// 13.4 -> 11.2 us, 256^2 FP64 13.7 -> 11.0 / 23.9 -> 20.9 us, 512^2 FP32
+// 25.9 -> 16.1 / 49.0 -> 51.4 us.  (512 FP32 columns in plan 0 batch 13%
+// faster, but their 32 elements per thread would set the register budget of
+// the multi-size group kernels, which mirror these defaults.)
+// 4096-point rows take plan 1 as well (4096^2 x-split rows FP64 / FP32:
+// 187-191 / 128-135 us); 4096-point columns (no x-split) plan 1 in FP64
+// (345 against 516 us) and plan 0 in FP32 (180 against 543 us).
+__host__ __device__ constexpr int default_variant(int prec, size_t n, bool row)
+{
+    return n == 1024   ? (prec == 64 ? 4 : 7)
+           : n == 2048 ? (prec == 64 ? (row ? 7 : 5) : (row ? 7 : 3))
+           : n == 4096 ? (row || prec == 64 ? 1 : 0)
+           : (n == 128 || n == 256 || n == 512) ? 1
+                                                : 0;
+}
+
 template <typename T, int N, int MODE, int V>
 int launch_row(const SplitDev *jobs, int njobs, size_t nrows, int iev, const void *tw,
                hipStream_t s)
 {
     using LP = P2Launch<T, N, false, V>;
+    // plans of lengths up to 512 that a new job starts with (the candidates
+    // of the longer ones fix their tiles)
+    if constexpr (N <= 512 && V == default_variant(sizeof(T) == 8 ? 64 : 32, N, true))
+        if (narrow_launch((nrows + LP::L - 1) / LP::L * njobs)) {
+            using NP = P2Launch<T, N, false, V, true>;
+            hipLaunchKernelGGL((k_row_sweep<T, N, MODE, V, false, true>),
+                               dim3((unsigned)((nrows + NP::L - 1) / NP::L), (unsigned)njobs),
+                               dim3(NP::THREADS), NP::LDS_BYTES, s, jobs, nrows, iev,
+                               (const c128 *)tw);
+            QSIM_HIP(hipGetLastError());
+            return QSIM_OK;
+        }
     auto fn = k_row_sweep<T, N, MODE, V, false>;
     if constexpr (N <= 1024)
         if (line_nt(N, (size_t)njobs * nrows * N * sizeof(cx<T>))) fn = k_row_sweep<T, N, MODE, V, true>;
@@ -856,6 +891,17 @@ int launch_col(const SplitDev *jobs, int njobs, size_t ncols, int ik, const void
                hipStream_t s)
 {
     using LP = P2Launch<T, N, true, V>;
+    if constexpr (N <= 512 && V == default_variant(sizeof(T) == 8 ? 64 : 32, N, false))
+        if (narrow_launch((R * ncols + LP::L - 1) / LP::L * njobs)) {
+            using NP = P2Launch<T, N, true, V, true>;
+            static_assert(NP::LDS_BYTES <= 65536, "narrow tiles need no LDS limit");
+            hipLaunchKernelGGL((k_col_sweep<T, N, V, false, R, true>),
+                               dim3((unsigned)((R * ncols + NP::L - 1) / NP::L), (unsigned)njobs),
+                               dim3(NP::THREADS), NP::LDS_BYTES, s, jobs, ncols, ik,
+                               (const c128 *)tw);
+            QSIM_HIP(hipGetLastError());
+            return QSIM_OK;
+        }
     auto fn = k_col_sweep<T, N, V, false, R>;
     if constexpr (N <= 1024)
         if (line_nt(N, (size_t)njobs * R * ncols * N * sizeof(cx<T>)))
@@ -912,29 +958,6 @@ int num_variants(size_t n)
                                                              : 1;
 }
 bool has_variants(size_t n) { return num_variants(n) > 1; }
-
-// Variants a new job starts with: the pairs the autotuner picked most often
-// on MI355X for single and batched jobs of these lengths (row variant by the
-// row length ny, column variant by the column length nx).  Fixed, so jobs that
-// are never tuned (request loops, batches) still take a fast pair and two
-// runs of one job always choose the same radix plans.
-// 128- to 512-point lines take the 8-per-thread plan (variant 1): measured
-// on MI355X per step, single job / 16 batched: 128^2 FP32 11.7 -> 9.6 /
-// 13.4 -> 11.2 us, 256^2 FP64 13.7 -> 11.0 / 23.9 -> 20.9 us, 512^2 FP32
-// 25.9 -> 16.1 / 49.0 -> 51.4 us.  (512 FP32 columns in plan 0 batch 13%
-// faster, but their 32 elements per thread would set the register budget of
-// the multi-size group kernels, which mirror these defaults.)
-// 4096-point rows take plan 1 as well (4096^2 x-split rows FP64 / FP32:
-// 187-191 / 128-135 us); 4096-point columns (no x-split) plan 1 in FP64
-// (345 against 516 us) and plan 0 in FP32 (180 against 543 us).
-__host__ __device__ constexpr int default_variant(int prec, size_t n, bool row)
-{
-    return n == 1024   ? (prec == 64 ? 4 : 7)
-           : n == 2048 ? (prec == 64 ? (row ? 7 : 5) : (row ? 7 : 3))
-           : n == 4096 ? (row || prec == 64 ? 1 : 0)
-           : (n == 128 || n == 256 || n == 512) ? 1
-                                                : 0;
-}
 
 // The x-split row sweep depends on the radix plan only (its lines per
 // workgroup are the R rows of a group): variants with the same plan share one

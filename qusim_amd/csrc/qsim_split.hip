@@ -574,13 +574,202 @@ __global__ void __launch_bounds__((P2Launch<T, N, true, V, NARROW>::THREADS))
 // ---------------------------------------------------------------- 1D job
 // Radix plan of the persistent 1D kernel per length.  A job is one workgroup
 // stepping its line on its own, so each step's chain of dependent work sets
-// the time: lengths 1024, 2048 and 4096 take four-pass plans with 8 elements
-// per thread (128 / 256 / 512 threads) instead of the 2D defaults (32 / 128 /
-// 256 threads).
+// the time: lengths of 128 to 4096 take plans with 8 elements per thread (16 to
+// 512 threads) instead of 16 to 32.
 template <typename T, int N>
 struct Split1DV {
-    static constexpr int V = (N == 1024 || N == 2048) ? 6 : (N == 4096 ? 1 : 0);
+    static constexpr int V = (N == 1024 || N == 2048)                            ? 6
+                             : (N == 128 || N == 256 || N == 512 || N == 4096) ? 1
+                                                                                 : 0;
 };
+
+// A line whose step constants stay in registers: the first power of every
+// butterfly's twiddle, and LDS exchanges that alternate between two buffers
+// (one barrier each; the buffer being written was read before the barrier of
+// the exchange in between).
+template <typename T, int N, typename P>
+struct KeptLine {
+    static constexpr int RA = P::RA_, RB = P::RB_, RC = P::RC_, RD = P::RD_, NP = P::NP;
+    static constexpr int E = P::E, TPL = P::TPL;
+    // first powers of passes 1 .. 3, forward and inverse
+    c128 f1[E / RB], f2[E / RC], f3[E / RD], i1[E], i2[E], i3[E / RA];
+    int t;
+    cx<T> *buf0, *buf1;
+
+    template <int R, int NS>
+    __device__ __forceinline__ void load(c128 *w, const c128 *__restrict__ tw)
+    {
+#pragma unroll
+        for (int u = 0; u < E / R; ++u)
+            w[u] = ld_g(tw + ((t + u * TPL) & (NS - 1)) * (N / (NS * R)));
+    }
+    __device__ __forceinline__ void init(int thread, cx<T> *lds, const c128 *__restrict__ tw)
+    {
+        t = thread;
+        buf0 = lds;
+        buf1 = lds + P::LS;
+        if constexpr (NP >= 2) load<RB, RA>(f1, tw);
+        if constexpr (NP >= 3) load<RC, RA * RB>(f2, tw);
+        if constexpr (NP == 4) load<RD, RA * RB * RC>(f3, tw);
+        if constexpr (NP == 2) load<RA, RB>(i1, tw);
+        if constexpr (NP == 3) {
+            load<RB, RC>(i1, tw);
+            load<RA, RC * RB>(i2, tw);
+        }
+        if constexpr (NP == 4) {
+            load<RC, RD>(i1, tw);
+            load<RB, RD * RC>(i2, tw);
+            load<RA, RD * RC * RB>(i3, tw);
+        }
+    }
+    // the powers by a product tree: a chain of 3 products for radix 8, not 6
+    template <int R, bool INV>
+    __device__ __forceinline__ void pass(cx<T> *v, const c128 *w1)
+    {
+#pragma unroll
+        for (int u = 0; u < E / R; ++u) {
+            c128 w[R];
+            w[1] = w1[u];
+#pragma unroll
+            for (int r = 2; r < R; ++r) w[r] = w[r / 2] * w[r - r / 2];
+#pragma unroll
+            for (int r = 1; r < R; ++r) {
+                const c128 x = cvt<double>(v[u * R + r]);
+                v[u * R + r] = cvt<T>(INV ? mulconj(x, w[r]) : x * w[r]);
+            }
+            dft_reg<T, R, INV>(v + u * R);
+        }
+    }
+    template <int R, bool INV>
+    __device__ __forceinline__ void first(cx<T> *v)
+    {
+#pragma unroll
+        for (int u = 0; u < E / R; ++u) dft_reg<T, R, INV>(v + u * R);
+    }
+    template <int R, int NS, int R2>
+    __device__ __forceinline__ void exchange(cx<T> *v, int which)
+    {
+        cx<T> *lds = which & 1 ? buf1 : buf0;
+#pragma unroll
+        for (int u = 0; u < E / R; ++u) {
+            const int j = t + u * TPL;
+            const int base = (j / NS) * NS * R + (j & (NS - 1));
+#pragma unroll
+            for (int r = 0; r < R; ++r) lds[P::template pad<R>(base + r * NS, 0)] = v[u * R + r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < E / R2; ++u)
+#pragma unroll
+            for (int r = 0; r < R2; ++r)
+                v[u * R2 + r] = lds[P::template pad<R>(P::template in_pos<R2>(t, u, r), 0)];
+    }
+    __device__ __forceinline__ void forward(cx<T> *v)
+    {
+        first<RA, false>(v);
+        if constexpr (NP >= 2) {
+            exchange<RA, 1, RB>(v, 0);
+            pass<RB, false>(v, f1);
+        }
+        if constexpr (NP >= 3) {
+            exchange<RB, RA, RC>(v, 1);
+            pass<RC, false>(v, f2);
+        }
+        if constexpr (NP == 4) {
+            exchange<RC, RA * RB, RD>(v, 2);
+            pass<RD, false>(v, f3);
+        }
+    }
+    // exchanges NP - 1 .. 2 NP - 3: an even number a step, so the next step
+    // starts with the buffer that this one did not end with
+    __device__ __forceinline__ void inverse(cx<T> *v)
+    {
+        if constexpr (NP == 1) {
+            first<RA, true>(v);
+        } else if constexpr (NP == 2) {
+            first<RB, true>(v);
+            exchange<RB, 1, RA>(v, 1);
+            pass<RA, true>(v, i1);
+        } else if constexpr (NP == 3) {
+            first<RC, true>(v);
+            exchange<RC, 1, RB>(v, 2);
+            pass<RB, true>(v, i1);
+            exchange<RB, RC, RA>(v, 3);
+            pass<RA, true>(v, i2);
+        } else {
+            first<RD, true>(v);
+            exchange<RD, 1, RC>(v, 3);
+            pass<RC, true>(v, i1);
+            exchange<RC, RD, RB>(v, 4);
+            pass<RB, true>(v, i2);
+            exchange<RB, RD * RC, RA>(v, 5);
+            pass<RA, true>(v, i3);
+        }
+    }
+};
+
+// The one-phase program (O2) of a line with 8 elements per thread: kinetic and
+// potential factors and twiddles stay in registers for all steps.  Reloaded
+// every step they were 170 KB of L2 reads a step at 4096 points, next to 12
+// barriers; what is left is LDS latency and FP64 issue, 6 exchanges a step.  us
+// a step: FP64 256 points 4.35 -> 1.63 (with 8 elements per thread instead of
+// 16), 2048 4.18 -> 3.18, 4096 6.42 -> 4.51; FP32 32 x 4096 5.66 -> 4.34, 8 x
+// 512 11.7 -> 2.1.  O4's five tables do not fit the registers and keep
+// k_split1d.
+template <typename T, int N>
+struct Kept1D {
+    using P = typename P2Cfg<T, N, Split1DV<T, N>::V>::Line;
+    static constexpr size_t LDS = 2 * (size_t)P::LS * sizeof(cx<T>);
+    static constexpr bool OK = P::E <= 8 && LDS <= 160 * 1024;
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__((Kept1D<T, N>::P::TPL))
+    k_split1d_kept(const SplitDev *__restrict__ jobs, Prog1D prog, size_t nsteps,
+                   const c128 *__restrict__ tw)
+{
+    using P = typename Kept1D<T, N>::P;
+    extern __shared__ unsigned char smem_raw[];
+    const SplitDev &J = jobs[blockIdx.x];
+    const int t = threadIdx.x;
+    constexpr int RA = P::RA_, RZ = P::RLAST;
+    KeptLine<T, N, P> line;
+    line.init(t, reinterpret_cast<cx<T> *>(smem_raw), tw);
+    cx<T> v[P::E];
+    c128 kp[P::E], ep[P::E];
+    c128 *psi = J.psi;
+    const c128 *e0 = J.ev[prog.ev0], *em = J.ev[prog.e[0]], *ez = J.ev[prog.ev_end];
+    const c128 *kt = J.kx[prog.k[0]];
+#pragma unroll
+    for (int u = 0; u < P::E / RA; ++u)
+#pragma unroll
+        for (int r = 0; r < RA; ++r) {
+            const int pos = P::template in_pos<RA>(t, u, r);
+            v[u * RA + r] = apply(conv<T>(ld_g(psi + pos)), ld_g(e0 + pos));
+            ep[u * RA + r] = ld_g(em + pos);
+        }
+#pragma unroll
+    for (int u = 0; u < P::E / RZ; ++u)
+#pragma unroll
+        for (int r = 0; r < RZ; ++r) kp[u * RZ + r] = ld_g(kt + P::template in_pos<RZ>(t, u, r));
+    for (size_t s = 0; s < nsteps; ++s) {
+        line.forward(v);
+#pragma unroll
+        for (int i = 0; i < P::E; ++i) v[i] = apply(v[i], kp[i]);
+        line.inverse(v);
+        if (s + 1 < nsteps) {
+#pragma unroll
+            for (int i = 0; i < P::E; ++i) v[i] = apply(v[i], ep[i]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < P::E / RA; ++u)
+#pragma unroll
+        for (int r = 0; r < RA; ++r) {
+            const int pos = P::template in_pos<RA>(t, u, r);
+            st_g(psi + pos, conv<double>(apply(v[u * RA + r], ld_g(ez + pos))));
+        }
+}
 
 template <typename T, int N>
 __global__ void __launch_bounds__((P2Cfg<T, N, Split1DV<T, N>::V>::Line::TPL))
@@ -919,6 +1108,16 @@ int launch_1d(const SplitDev *jobs, int njobs, const Prog1D &prog, size_t nsteps
               hipStream_t s)
 {
     using P = typename P2Cfg<T, N, Split1DV<T, N>::V>::Line;
+    if constexpr (Kept1D<T, N>::OK)
+        if (prog.nph == 1) {
+            auto fn = k_split1d_kept<T, N>;
+            constexpr size_t lds = Kept1D<T, N>::LDS;
+            QSIM_TRY(lds_limit((const void *)fn, lds));
+            hipLaunchKernelGGL(fn, dim3((unsigned)njobs), dim3(P::TPL), lds, s, jobs, prog, nsteps,
+                               (const c128 *)tw);
+            QSIM_HIP(hipGetLastError());
+            return QSIM_OK;
+        }
     auto fn = k_split1d<T, N>;
     const size_t lds = (size_t)P::LS * sizeof(cx<T>);
     QSIM_TRY(lds_limit((const void *)fn, lds));

@@ -49,7 +49,8 @@ struct At {
     c128 get(int e) const { return x.at(e); }
     void set(int e, c128 v) const { x.at(e) = v; }
 };
-static void prime(std::vector<c128> &x, const MixPass &p, const std::vector<c128> &tw)
+template <int M>
+static void prime_m(std::vector<c128> &x, const MixPass &p, const std::vector<c128> &tw)
 {
     std::vector<c128> y(x.size());
     std::vector<int> hit(x.size(), 0);
@@ -58,9 +59,10 @@ static void prime(std::vector<c128> &x, const MixPass &p, const std::vector<c128
         if ((p.R - 1) * mix_mod(p, j) * p.tws >= tlen || (p.R - 1) * p.nb >= tlen) ++failures;
         for (int k = 1; k <= H; ++k) mix_prime_pair(p, tw.data(), j, k, At{x});
     }
+    const int dm = (H + M) / M;
     for (int j = 0; j < p.nb; ++j)
-        for (int m = 0; m <= H; ++m)
-            mix_prime_out(p, tw.data(), j, m, At{x}, [&](int e, c128 v) {
+        for (int m = 0; m < dm; ++m)
+            mix_prime_out<M>(p, tw.data(), j, m, dm, At{x}, [&](int e, c128 v) {
                 y.at(e) = v;
                 ++hit[e];
             });
@@ -71,6 +73,14 @@ static void prime(std::vector<c128> &x, const MixPass &p, const std::vector<c128
     for (int h : hit)
         if (h != 1) ++failures;
     x.swap(y);
+}
+
+static void prime(std::vector<c128> &x, const MixPass &p, const std::vector<c128> &tw)
+{
+    static int turn = 0;
+    if (++turn % 3 == 0) prime_m<1>(x, p, tw);
+    else if (turn % 3 == 1) prime_m<2>(x, p, tw);
+    else prime_m<4>(x, p, tw);
 }
 
 static void transform(std::vector<c128> &x, const MixPass *f, int nf, const std::vector<c128> &tw)

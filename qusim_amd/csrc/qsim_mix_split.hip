@@ -11,12 +11,26 @@ namespace qsim {
 
 constexpr int kMix1dThreads = 768;
 
+// Lines are read once a sweep: from 6 MiB a sweep on, non-temporal loads keep
+// E_V and the tables in L2 (1000 x 1000: 34.0 -> 32.5 us a step, 1200 x
+// 1200 61.8 -> 60.4; 300 x 300 would lose 4%).
+template <bool NT>
+__device__ __forceinline__ c128 ld_psi(const c128 *p)
+{
+    if constexpr (NT) return ld_nt(p);
+    else return ld_g(p);
+}
+static bool psi_nt(const MixPlan &p, size_t nlines)
+{
+    return (size_t)p.n * nlines * sizeof(c128) >= ((size_t)6 << 20);
+}
+
 // Row and column sweeps: 32 B of psi and 16 B of E_V per point move once.  At
-// 1000 x 1000 a step takes 34 us (the unfused order's 8 passes: 300 us) and at 1500 x 1500 77 us (2.3 TB/s of the 80 B);
+// 1000 x 1000 a step takes 32 us (the unfused order's 8 passes: 300 us) and at 1500 x 1500 77 us (2.3 TB/s of the 80 B);
 // below that the chain of one workgroup's passes bounds the sweeps (750 x 600:
 // 27 us a step, each wave waits for 75% of its cycles), above it the LDS
 // exchanges.
-template <int MODE>
+template <int MODE, bool NT>
 __global__ void __launch_bounds__(kMixMaxThreads)
     k_mix_row(c128 *psi, const c128 *ev, int twice, unsigned nrows, MixPlan p, MixDims d,
               const c128 *__restrict__ tw)
@@ -35,7 +49,7 @@ __global__ void __launch_bounds__(kMixMaxThreads)
         if (active) store_nt(psi + (unsigned)m, v);
         return v;
     };
-    auto load_inv = [&](int, int m, c128, c128) { return mix_swap(ld_g(psi + (unsigned)m)); };
+    auto load_inv = [&](int, int m, c128, c128) { return mix_swap(ld_psi<NT>(psi + (unsigned)m)); };
     if constexpr (MODE == SW_FIRST) {
         mix_one(
             w, p,
@@ -59,6 +73,7 @@ __global__ void __launch_bounds__(kMixMaxThreads)
     }
 }
 
+template <bool NT>
 __global__ void __launch_bounds__(kMixMaxThreads)
     k_mix_col(c128 *psi, const c128 *kx, const c128 *ky, double scale, unsigned ncols, MixPlan p,
               MixDims d, const c128 *__restrict__ tw)
@@ -73,7 +88,7 @@ __global__ void __launch_bounds__(kMixMaxThreads)
     const c128 kyj = ld_g(ky + c);
     auto at = [&](int m) { return psi + (size_t)((unsigned)m * (size_t)ncols); };
     mix_two(
-        w, p, [&](int, int m, c128, c128) { return ld_g(at(m)); },
+        w, p, [&](int, int m, c128, c128) { return ld_psi<NT>(at(m)); },
         [&](int, int m) { return ld_g(kx + (unsigned)m); },
         [&](int, int, c128 v, c128 k) { return mix_swap(v * k * kyj); },
         [&](int, int m, c128 v, c128) {
@@ -132,8 +147,11 @@ static int launch_row(const SplitDev &job, size_t nrows, int iev, bool twice,
                       const MixPlan &p, const void *tw, hipStream_t s)
 {
     const MixShape sh = mix_shape(p, nrows, sizeof(c128), false);
-    QSIM_TRY(lds_limit((const void *)k_mix_row<MODE>, kMixMaxLds));
-    hipLaunchKernelGGL(k_mix_row<MODE>, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, job.psi,
+    auto fn = k_mix_row<MODE, false>;
+    if constexpr (MODE != SW_FIRST)
+        if (psi_nt(p, nrows)) fn = k_mix_row<MODE, true>;
+    QSIM_TRY(lds_limit((const void *)fn, kMixMaxLds));
+    hipLaunchKernelGGL(fn, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, job.psi,
                        job.ev[iev], (int)twice, (unsigned)nrows, p, sh.d, (const c128 *)tw);
     QSIM_HIP(hipGetLastError());
     return QSIM_OK;
@@ -151,8 +169,9 @@ int mix_col_sweep(const SplitDev &job, size_t ncols, int ik, const MixPlan &p, c
                   hipStream_t s)
 {
     const MixShape sh = mix_shape(p, ncols, sizeof(c128), true);
-    QSIM_TRY(lds_limit((const void *)k_mix_col, kMixMaxLds));
-    hipLaunchKernelGGL(k_mix_col, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, job.psi,
+    auto fn = psi_nt(p, ncols) ? k_mix_col<true> : k_mix_col<false>;
+    QSIM_TRY(lds_limit((const void *)fn, kMixMaxLds));
+    hipLaunchKernelGGL(fn, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, job.psi,
                        job.kx[ik], job.ky[ik], 1.0 / ((double)p.n * (double)ncols),
                        (unsigned)ncols, p, sh.d, (const c128 *)tw);
     QSIM_HIP(hipGetLastError());

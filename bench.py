@@ -177,11 +177,11 @@ def probe_kernels(rv, cv, xs):
     are instantiated per radix plan: row variants 1 and 5 run plan 0, 3 runs
     2, 7 runs 6."""
     if xs == 1:
-        return (("row_sweep", r"k_row_sweep<double, 1024, 1, %d, (true|false)>" % rv),
-                ("col_sweep", r"k_col_sweep<double, 1024, %d, (true|false), 1>" % cv))
+        return (("row_sweep", r"k_row_sweep<double, 1024, 1, %d, (true|false)(, false)?>" % rv),
+                ("col_sweep", r"k_col_sweep<double, 1024, %d, (true|false), 1(, false)?>" % cv))
     plan = {1: 0, 5: 0, 3: 2, 7: 6}.get(rv, rv)
     return (("row_sweep", r"k_row_sweep_x<double, 1024, 1, %d, (true|false), %d>" % (plan, xs)),
-            ("col_sweep", r"k_col_sweep<double, %d, %d, (true|false), %d>" % (1024 // xs, cv, xs)))
+            ("col_sweep", r"k_col_sweep<double, %d, %d, (true|false), %d(, false)?>" % (1024 // xs, cv, xs)))
 
 
 def batch_probe(steps, njobs, variants, n=1024):

@@ -13,7 +13,8 @@ constexpr int kMix1dThreads = 768;
 
 // Lines are read once a sweep: from 6 MiB a sweep on, non-temporal loads keep
 // E_V and the tables in L2 (1000 x 1000: 34.0 -> 32.5 us a step, 1200 x
-// 1200 61.8 -> 60.4; 300 x 300 would lose 4%).
+// 1200 61.8 -> 60.4, both timed with two entries' products as higher twiddle
+// powers; 300 x 300 would lose 4%).
 template <bool NT>
 __device__ __forceinline__ c128 ld_psi(const c128 *p)
 {
@@ -26,9 +27,11 @@ static bool psi_nt(const MixPlan &p, size_t nlines)
 }
 
 // Row and column sweeps: 32 B of psi and 16 B of E_V per point move once.  At
-// 1000 x 1000 a step takes 32 us (the unfused order's 8 passes: 300 us) and at 1500 x 1500 77 us (2.3 TB/s of the 80 B);
+// 1000 x 1000 a step takes 32 us (the unfused order's 8 passes: 300 us) and at
+// 1500 x 1500 82 us (2.2 TB/s of the 80 B);
 // below that the chain of one workgroup's passes bounds the sweeps (750 x 600:
-// 27 us a step, each wave waits for 75% of its cycles), above it the LDS
+// 27 us a step, waves wait for 77% of their cycles in the row sweep and 62% in
+// the column sweep), above it the LDS
 // exchanges.
 template <int MODE, bool NT>
 __global__ void __launch_bounds__(kMixMaxThreads)
@@ -97,11 +100,10 @@ __global__ void __launch_bounds__(kMixMaxThreads)
         });
 }
 
-// All steps of one line: 768 threads at most, so that
-// 168 registers are left (at 128 the wide radices spill: 1000 points 6.2
-// against 5.3 us a step).  Bound by the latency of its passes: a step of n =
-// 1000 is 6 of about 0.9 us, half of it LDS and barriers; the unfused order's
-// 7 launches took 66 us.
+// All steps of one line: 768 threads at most, so that 168 registers are left (at
+// 128 the wide radices spilled: 1000 points 6.2 against 5.3 us a step when
+// timed).  Bound by the latency of its passes: a step of n = 1000 is 6 of about
+// 0.9 us (an O4 stage 5.6 us); the unfused order's 7 launches took 66 us.
 __global__ void __launch_bounds__(kMix1dThreads)
     k_mix_1d(SplitDev J, Prog1D prog, size_t nsteps, double scale, MixPlan p, MixDims d, int nreal,
              const c128 *__restrict__ tw)

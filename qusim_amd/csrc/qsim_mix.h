@@ -355,8 +355,9 @@ struct MixDft<15> {
 
 // Twiddles of one butterfly, w^r for r < R, each a rounded table entry read
 // where it is used (the table stays in LDS).  With w^4 + q and w^8 + q as
-// products of two entries 1000 points cost 315 us instead of 333 (O4, 20 steps)
-// at an error of 1.2e-14 instead of 0.94e-14 (the generic kernel's: 0.99e-14).
+// products of two entries 1000 points cost 315 us instead of 333 (O4, 20 steps),
+// but after 60 transform pairs (on the CPU, 51 lengths, the same inputs) the
+// error was 1.36 times that of direct sums in the mean instead of 1.19.
 template <int R>
 struct MixTw {
     const c128 *t;

@@ -729,10 +729,13 @@ inline void mix_split(int n, int maxr, int depth, double work, double cost, int 
 // `work`: line elements that a CU holds at a time.  false when n is not a
 // composite number with prime factors of at most 13, 4 <= n <= kMixMaxLen, or
 // any number with a larger prime factor whose line fits LDS twice (mix_fits:
-// up to 3150 points).
+// up to 3150 points).  *out is then an empty plan (n = 0): callers keep it as
+// "no mixed-radix line here".
 bool mix_fits(const MixPlan &p);
-inline bool mix_plan(size_t n, double work, MixPlan *p)
+inline bool mix_plan(size_t n, double work, MixPlan *out)
 {
+    *out = MixPlan{};
+    MixPlan plan{}, *p = &plan;
     if (n < 4 || n > (size_t)kMixMaxLen) return false;
     int primes[kMixMaxPasses], np = 0, s = (int)n;
     for (int q = 17; q <= s; q += 2)
@@ -780,7 +783,9 @@ inline bool mix_plan(size_t n, double work, MixPlan *p)
             ns *= R;
         }
     }
-    return mix_fits(*p);
+    if (!mix_fits(*p)) return false;
+    *out = plan;
+    return true;
 }
 
 // Elements of `nlines` lines of n points that one of 256 CUs holds at a time:

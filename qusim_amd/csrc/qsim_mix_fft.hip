@@ -37,6 +37,7 @@ template <typename T, bool INV>
 static int launch(const FftAxis &a, const void *in, void *out, double scale, hipStream_t s)
 {
     const MixShape sh = mix_shape(a.mix, a.nlines, sizeof(cx<T>), a.S > 1);
+    QSIM_CHECK(sh.d.nt > 0, "mixed-radix transform: launch shape");
     auto fn = k_fft_mix<T, INV>;
     QSIM_TRY(lds_limit((const void *)fn, kMixMaxLds));
     hipLaunchKernelGGL(fn, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, (const cx<T> *)in,

@@ -64,34 +64,39 @@ __host__ __device__ constexpr int mix_k(int R)
 __host__ __device__ __forceinline__ int mix_slot(int e, int sh) { return e + (e >> sh); }
 
 // ------------------------------------------------------------- butterflies
+// A rounded constant repeats its rounding in every transform, and over the
+// steps of an evolution that grows with their number, not with its root.
+// Constants whose rounding showed (those of 3, 5, 8, 9 and 11 points) come as
+// the double and the low part that the rounding took off; the low part goes
+// into the addend of a product's fma, where the rounding that follows still
+// moves by it, never onto a value alone.  7 and 13 points: MixPrime.
+
 // cos and sin of 2 pi k / P, k = 1 .. (P-1)/2
 template <int P>
 struct MixC;
-template <>
-struct MixC<3> {
-    static constexpr double c[1] = {-0.5};
-    static constexpr double s[1] = {0.86602540378443864676};
-};
-template <>
-struct MixC<5> {
-    static constexpr double c[2] = {0.30901699437494742410, -0.80901699437494742410};
-    static constexpr double s[2] = {0.95105651629515357212, 0.58778525229247312917};
-};
 template <>
 struct MixC<7> {
     static constexpr double c[3] = {0.62348980185873353053, -0.22252093395631440429,
                                     -0.90096886790241912624};
     static constexpr double s[3] = {0.78183148246802980871, 0.97492791218182360702,
                                     0.43388373911755812048};
+    static constexpr bool LOW = false;
 };
 template <>
 struct MixC<11> {
     static constexpr double c[5] = {0.84125353283118116886, 0.41541501300188642553,
-                                    -0.14231483827328514044, -0.65486073394528506407,
+                                    -0.14231483827328514044, -0.65486073394528506406,
                                     -0.95949297361449738988};
-    static constexpr double s[5] = {0.54064081745559758211, 0.90963199535451837140,
+    static constexpr double s[5] = {0.54064081745559758211, 0.90963199535451837141,
                                     0.98982144188093273238, 0.75574957435425828377,
                                     0.28173255684142969771};
+    static constexpr bool LOW = true;
+    static constexpr double cl[5] = {-3.6647285149858677e-17, -9.5552123437671800e-18,
+                                     3.1334476506295326e-18, 3.6553153571046389e-17,
+                                     -2.1239679343678974e-17};
+    static constexpr double sl[5] = {2.6677788920071333e-17, 4.1301477016464232e-17,
+                                     4.8155296856458766e-17, 1.4869519672512073e-17,
+                                     2.6676302681156600e-17};
 };
 template <>
 struct MixC<13> {
@@ -101,6 +106,7 @@ struct MixC<13> {
     static constexpr double s[6] = {0.46472317204376854566, 0.82298386589365639458,
                                     0.99270887409805399280, 0.93501624268541482344,
                                     0.66312265824079520238, 0.23931566428755776714};
+    static constexpr bool LOW = false;
 };
 
 __host__ __device__ __forceinline__ c128 mix_mi(c128 a) { return mk(a.y, -a.x); }  // -i a
@@ -116,6 +122,20 @@ __host__ __device__ __forceinline__ c128 mix_fms(c128 a, c128 b, c128 c)
     return mk(fma(b.y, c.y, fma(-b.x, c.x, a.x)), fma(-b.y, c.x, fma(-b.x, c.y, a.y)));
 }
 
+// a w with w = h + l, l the low part
+__host__ __device__ __forceinline__ c128 mix_mul(c128 a, c128 h, c128 l)
+{
+    return mix_fma(a * l, a, h);
+}
+
+// a / n by s = 1 / n, sl = mix_recip_lo(n): the rounding of 1 / n alone grew to
+// 5e-15 over 60 steps of 243 or 850 points
+__host__ __device__ __forceinline__ c128 mix_scale(c128 a, double s, double sl)
+{
+    return mk(fma(a.x, s, a.x * sl), fma(a.y, s, a.y * sl));
+}
+inline double mix_recip_lo(double n) { return fma(-(1.0 / n), n, 1.0) / n; }
+
 // An R-point butterfly starts with sums and differences of pairs: pair(i, h)
 // is element h (0, 1) of pair i.  rest() takes the sums in the first and the
 // differences in the second places of the pairs and finishes the transform;
@@ -125,6 +145,9 @@ struct MixDft;
 
 // An odd prime: X_m = x0 + sum_k (x_k + x_{P-k}) cos(2 pi k m / P)
 //                        - i sum_k (x_k - x_{P-k}) sin(2 pi k m / P)
+// The roundings of 7 and 13 points' constants left 60 steps of 343 to 3003
+// points at 0.9 to 1.1 times the error of direct sums, so they take none of
+// the low parts' instructions.
 template <int P>
 struct MixPrime {
     static constexpr int PAIRS = (P - 1) / 2;
@@ -143,37 +166,73 @@ struct MixPrime {
         v[0] = s0;
 #pragma unroll
         for (int m = 1; m <= H; ++m) {
-            c128 e = x0, o = mk(0.0, 0.0);
+            constexpr bool LOW = MixC<P>::LOW;
+            c128 e = LOW ? mk(0.0, 0.0) : x0, o = mk(0.0, 0.0);
+            if constexpr (LOW) {
+#pragma unroll
+                for (int k = 1; k <= H; ++k) {
+                    const int q = (k * m) % P, i = (q <= H ? q : P - q) - 1;
+                    const double c = MixC<P>::cl[i];
+                    const double s = q <= H ? MixC<P>::sl[i] : -MixC<P>::sl[i];
+                    e = k == 1 ? mk(c * a[0].x, c * a[0].y)
+                               : mk(fma(c, a[k - 1].x, e.x), fma(c, a[k - 1].y, e.y));
+                    o = k == 1 ? mk(s * b[0].x, s * b[0].y)
+                               : mk(fma(s, b[k - 1].x, o.x), fma(s, b[k - 1].y, o.y));
+                }
+            }
 #pragma unroll
             for (int k = 1; k <= H; ++k) {
-                const int q = (k * m) % P;
-                const double c = MixC<P>::c[(q <= H ? q : P - q) - 1];
-                const double s = q <= H ? MixC<P>::s[q - 1] : -MixC<P>::s[P - q - 1];
+                const int q = (k * m) % P, i = (q <= H ? q : P - q) - 1;
+                const double c = MixC<P>::c[i], s = q <= H ? MixC<P>::s[i] : -MixC<P>::s[i];
                 e = mk(fma(c, a[k - 1].x, e.x), fma(c, a[k - 1].y, e.y));
-                o = k == 1 ? mk(s * b[0].x, s * b[0].y)
-                           : mk(fma(s, b[k - 1].x, o.x), fma(s, b[k - 1].y, o.y));
+                o = k == 1 && !LOW ? mk(s * b[0].x, s * b[0].y)
+                                   : mk(fma(s, b[k - 1].x, o.x), fma(s, b[k - 1].y, o.y));
             }
+            if constexpr (LOW) e = x0 + e;
             const c128 io = mix_mi(o);
             v[m] = e + io;
             v[P - m] = e - io;
         }
     }
 };
-template <> struct MixDft<3> : MixPrime<3> {};
-// 5: the cosines' mean is -1/4 exactly, so the even part takes one rounded
-// constant, sqrt(5) / 4, instead of two.
+// 3: the cosine is -1/2 exactly.
 template <>
-struct MixDft<5> : MixPrime<5> {
+struct MixDft<3> {
+    static constexpr int PAIRS = 1;
+    static __host__ __device__ constexpr int pair(int, int h) { return 1 + h; }
     static __host__ __device__ __forceinline__ void rest(c128 *v)
     {
-        constexpr double k = 0.55901699437494742410, s1 = MixC<5>::s[0], s2 = MixC<5>::s[1];
-        const c128 x0 = v[0], a = v[1] + v[2], d = v[1] - v[2], b1 = v[4], b2 = v[3];
-        const c128 t = mk(fma(-0.25, a.x, x0.x), fma(-0.25, a.y, x0.y));
-        const c128 e1 = mk(fma(k, d.x, t.x), fma(k, d.y, t.y));
-        const c128 e2 = mk(fma(-k, d.x, t.x), fma(-k, d.y, t.y));
-        const c128 o1 = mk(fma(s1, b1.y, s2 * b2.y), -fma(s1, b1.x, s2 * b2.x));   // -i o
-        const c128 o2 = mk(fma(s2, b1.y, -(s1 * b2.y)), fma(-s2, b1.x, s1 * b2.x));
+        constexpr double s = 0.86602540378443864676, sl = 5.0175421109034514e-17;
+        const c128 x0 = v[0], a = v[1], b = v[2];
+        const c128 e = mk(fma(-0.5, a.x, x0.x), fma(-0.5, a.y, x0.y));
+        const c128 o = mk(fma(s, b.y, sl * b.y), -fma(s, b.x, sl * b.x));   // -i o
         v[0] = x0 + a;
+        v[1] = e + o;
+        v[2] = e - o;
+    }
+};
+// 5: the cosines' low parts are -q and q; the second sine's, a fifteenth of a
+// unit, is left out.
+template <>
+struct MixDft<5> {
+    static constexpr int PAIRS = 2;
+    static __host__ __device__ constexpr int pair(int i, int h) { return h ? 4 - i : i + 1; }
+    static __host__ __device__ __forceinline__ void rest(c128 *v)
+    {
+        constexpr double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;
+        constexpr double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;
+        constexpr double q = 2.7160576018412531e-17, l1 = 4.0934500900087295e-17;
+        const c128 x0 = v[0], a1 = v[1], a2 = v[2], b1 = v[4], b2 = v[3];
+        const c128 lo = q * (a2 - a1);
+        const c128 e1 = mk(fma(c2, a2.x, x0.x) + fma(c1, a1.x, lo.x),
+                           fma(c2, a2.y, x0.y) + fma(c1, a1.y, lo.y));
+        const c128 e2 = mk(fma(c1, a2.x, x0.x) + fma(c2, a1.x, -lo.x),
+                           fma(c1, a2.y, x0.y) + fma(c2, a1.y, -lo.y));
+        const c128 o1 = mk(fma(s1, b1.y, fma(s2, b2.y, l1 * b1.y)),
+                           -fma(s1, b1.x, fma(s2, b2.x, l1 * b1.x)));   // -i o
+        const c128 o2 = mk(fma(s2, b1.y, -fma(s1, b2.y, l1 * b2.y)),
+                           fma(-s2, b1.x, fma(s1, b2.x, l1 * b2.x)));
+        v[0] = x0 + (a1 + a2);
         v[1] = e1 + o1;
         v[4] = e1 - o1;
         v[2] = e2 + o2;
@@ -232,10 +291,12 @@ struct MixDft<8> {
     static __host__ __device__ constexpr int pair(int i, int h) { return i + 4 * h; }
     static __host__ __device__ __forceinline__ void rest(c128 *v)
     {
-        constexpr double h = 0.70710678118654752440;
+        auto mul = [](double x) {   // by sqrt(1/2)
+            return fma(0.70710678118654752440, x, -4.8336466567264567e-17 * x);
+        };
         c128 u[4] = {v[0], v[1], v[2], v[3]};
-        c128 w[4] = {v[4], mk(h * (v[5].x + v[5].y), h * (v[5].y - v[5].x)), mix_mi(v[6]),
-                     mk(h * (v[7].y - v[7].x), -h * (v[7].x + v[7].y))};
+        c128 w[4] = {v[4], mk(mul(v[5].x + v[5].y), mul(v[5].y - v[5].x)), mix_mi(v[6]),
+                     mk(mul(v[7].y - v[7].x), -mul(v[7].x + v[7].y))};
         mix_dft<4>(u);
         mix_dft<4>(w);
 #pragma unroll
@@ -251,10 +312,13 @@ struct MixDft<9> {
     static __host__ __device__ constexpr int pair(int i, int h) { return 3 + i + 3 * h; }
     static __host__ __device__ __forceinline__ void rest(c128 *v)
     {
-        // w_9^1, w_9^2, w_9^4
+        // w_9^1, w_9^2, w_9^4 and their low parts
         constexpr c128 w1 = {0.76604444311897803520, -0.64278760968653932632},
                        w2 = {0.17364817766693034885, -0.98480775301220805937},
-                       w4 = {-0.93969262078590838405, -0.34202014332566873304};
+                       w4 = {-0.93969262078590838405, -0.34202014332566873304},
+                       l1 = {2.1750711742081045e-17, 3.6596079007909491e-17},
+                       l2 = {-1.0090493350843633e-17, -3.9051088757992981e-17},
+                       l4 = {4.3850932840020416e-17, -2.0136016534644645e-17};
         c128 t[3][3];
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
@@ -262,10 +326,10 @@ struct MixDft<9> {
             for (int a = 0; a < 3; ++a) t[b][a] = v[3 * a + b];
             MixDft<3>::rest(t[b]);
         }
-        t[1][1] = t[1][1] * w1;
-        t[1][2] = t[1][2] * w2;
-        t[2][1] = t[2][1] * w2;
-        t[2][2] = t[2][2] * w4;
+        t[1][1] = mix_mul(t[1][1], w1, l1);
+        t[1][2] = mix_mul(t[1][2], w2, l2);
+        t[2][1] = mix_mul(t[2][1], w2, l2);
+        t[2][2] = mix_mul(t[2][2], w4, l4);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             c128 u[3] = {t[0][k], t[1][k], t[2][k]};
@@ -697,10 +761,14 @@ __device__ __forceinline__ void mix_two(MixWg<T> &w, const MixPlan &p, In in, Pr
 // points (4.2, 3.8 and 3.8), and differ by less than 5% on grids.
 inline double mix_cost(int R, double work)
 {
-    // butterfly, twiddles and index arithmetic
+    // butterfly, twiddles and index arithmetic; of the low parts' instructions
+    // only those of 9, 11 and 15 points are in (1920 x 1920 646 -> 603 us for 5
+    // steps, 120^3 Born 582 -> 532, 972 points 443 -> 373, the rest within 1%):
+    // with all, plans have more and smaller radices, at 900 x 900 177 us instead
+    // of 163, and one transform is 1.2% further off in the mean
     const int instr = R == 2 ? 40 : R == 3 ? 60 : R == 4 ? 64 : R == 5 ? 96 : R == 6 ? 112
-                      : R == 7 ? 146 : R == 8 ? 148 : R == 9 ? 212 : R == 10 ? 212
-                      : R == 11 ? 274 : R == 12 ? 240 : R == 13 ? 348 : R == 14 ? 320 : 340;
+                      : R == 7 ? 146 : R == 8 ? 148 : R == 9 ? 240 : R == 10 ? 212
+                      : R == 11 ? 384 : R == 12 ? 240 : R == 13 ? 348 : R == 14 ? 320 : 386;
     const double waves = work / (256.0 * R);
     return 700 + 4 * instr * (waves > 1 ? waves : 1);
 }

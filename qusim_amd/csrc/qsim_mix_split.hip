@@ -78,8 +78,8 @@ __global__ void __launch_bounds__(kMixMaxThreads)
 
 template <bool NT>
 __global__ void __launch_bounds__(kMixMaxThreads)
-    k_mix_col(c128 *psi, const c128 *kx, const c128 *ky, double scale, unsigned ncols, MixPlan p,
-              MixDims d, const c128 *__restrict__ tw)
+    k_mix_col(c128 *psi, const c128 *kx, const c128 *ky, double scale, double scale_lo,
+              unsigned ncols, MixPlan p, MixDims d, const c128 *__restrict__ tw)
 {
     extern __shared__ unsigned char smem_raw[];
     MixWg<double> w = mix_begin<double>(smem_raw, p, d, tw);
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(kMixMaxThreads)
         [&](int, int m) { return ld_g(kx + (unsigned)m); },
         [&](int, int, c128 v, c128 k) { return mix_swap(v * k * kyj); },
         [&](int, int m, c128 v, c128) {
-            if (active) store_nt(at(m), mix_swap(v) * scale);
+            if (active) store_nt(at(m), mix_scale(mix_swap(v), scale, scale_lo));
             return v;
         });
 }
@@ -105,8 +105,8 @@ __global__ void __launch_bounds__(kMixMaxThreads)
 // timed).  Bound by the latency of its passes: a step of n = 1000 is 6 of about
 // 0.9 us (an O4 stage 5.6 us); the unfused order's 7 launches took 66 us.
 __global__ void __launch_bounds__(kMix1dThreads)
-    k_mix_1d(SplitDev J, Prog1D prog, size_t nsteps, double scale, MixPlan p, MixDims d, int nreal,
-             const c128 *__restrict__ tw)
+    k_mix_1d(SplitDev J, Prog1D prog, size_t nsteps, double scale, double scale_lo,
+             MixPlan p, MixDims d, int nreal, const c128 *__restrict__ tw)
 {
     extern __shared__ unsigned char smem_raw[];
     MixWg<double> w = mix_begin<double>(smem_raw, p, d, tw);
@@ -133,12 +133,12 @@ __global__ void __launch_bounds__(kMix1dThreads)
             auto evm = [&](int, int m) { return ld_g(ev + m); };
             if (last)
                 mix_pass<MIX_LAST, 10>(w, mix_last(p, true), evm, [&](int, int m, c128 v, c128 e) {
-                    if (m < nreal) st_g(psi + m, mix_swap(v) * scale * e);
+                    if (m < nreal) st_g(psi + m, mix_scale(mix_swap(v), scale, scale_lo) * e);
                     return v;
                 });
             else
                 mix_pass<MIX_TURN, 10>(w, mix_last(p, true), evm, [&](int, int, c128 v, c128 e) {
-                    v = mix_swap(v) * scale * e;
+                    v = mix_scale(mix_swap(v), scale, scale_lo) * e;
                     return twice ? v * e : v;
                 });
         }
@@ -173,9 +173,10 @@ int mix_col_sweep(const SplitDev &job, size_t ncols, int ik, const MixPlan &p, c
     const MixShape sh = mix_shape(p, ncols, sizeof(c128), true);
     auto fn = psi_nt(p, ncols) ? k_mix_col<true> : k_mix_col<false>;
     QSIM_TRY(lds_limit((const void *)fn, kMixMaxLds));
+    const double n = (double)p.n * (double)ncols;
     hipLaunchKernelGGL(fn, dim3(sh.d.blocks), dim3(sh.d.nt), sh.lds, s, job.psi,
-                       job.kx[ik], job.ky[ik], 1.0 / ((double)p.n * (double)ncols),
-                       (unsigned)ncols, p, sh.d, (const c128 *)tw);
+                       job.kx[ik], job.ky[ik], 1.0 / n, mix_recip_lo(n), (unsigned)ncols, p,
+                       sh.d, (const c128 *)tw);
     QSIM_HIP(hipGetLastError());
     return QSIM_OK;
 }
@@ -186,8 +187,8 @@ int mix_run_1d(const SplitDev &job, const Prog1D &prog, size_t nsteps, const Mix
     const MixShape sh = mix_shape_of(p, 0, 1, sizeof(c128), kMixMaxLds);
     QSIM_CHECK(sh.d.nt > 0 && sh.d.nt <= kMix1dThreads, "1D line: launch shape");
     QSIM_TRY(lds_limit((const void *)k_mix_1d, kMixMaxLds));
-    hipLaunchKernelGGL(k_mix_1d, dim3(1), dim3(sh.d.nt), sh.lds, s, job, prog, nsteps, 1.0 / p.n, p, sh.d,
-                       (int)nreal, (const c128 *)tw);
+    hipLaunchKernelGGL(k_mix_1d, dim3(1), dim3(sh.d.nt), sh.lds, s, job, prog, nsteps, 1.0 / p.n,
+                       mix_recip_lo(p.n), p, sh.d, (int)nreal, (const c128 *)tw);
     QSIM_HIP(hipGetLastError());
     return QSIM_OK;
 }

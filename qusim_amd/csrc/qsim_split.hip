@@ -622,7 +622,6 @@ struct KeptLine {
             load<RA, RD * RC * RB>(i3, tw);
         }
     }
-    // the powers by a product tree: a chain of 3 products for radix 8, not 6
     template <int R, bool INV>
     __device__ __forceinline__ void pass(cx<T> *v, const c128 *w1)
     {
@@ -630,8 +629,7 @@ struct KeptLine {
         for (int u = 0; u < E / R; ++u) {
             c128 w[R];
             w[1] = w1[u];
-#pragma unroll
-            for (int r = 2; r < R; ++r) w[r] = w[r / 2] * w[r - r / 2];
+            twiddle_powers<R>(w);
 #pragma unroll
             for (int r = 1; r < R; ++r) {
                 const c128 x = cvt<double>(v[u * R + r]);

@@ -810,12 +810,13 @@ int epsilon_for(qsim_born_job *j, int e, double *eps)
             const c128 ve = ve_at(idx);
             v[0] = ve.y;
             v[1] = abs2(ve);
-        }));
+        }, red::kOneBlockDiv));
         minEps = 0.5 * r[1] / (-r[0]);
     } else {
         double m2 = 0;
         QSIM_TRY(red::reduce_ext<true>(n, nullptr, 0.0, &m2,
-                                       [=] __device__(size_t idx) { return abs2(ve_at(idx)); }));
+                                       [=] __device__(size_t idx) { return abs2(ve_at(idx)); },
+                                       red::kOneBlockDiv));
         minEps = std::sqrt(m2);
     }
     if (*eps < minEps) *eps = minEps;
@@ -1324,7 +1325,7 @@ int qsim_hip_born_xsection(qsim_born_job *j, int e, double cosx, double cosy, do
             const c128 t = (tot_at(idx, ix, iy, iz) * V[idx].x) * mk(cs, sn);
             v[0] = t.x;
             v[1] = t.y;
-        }));
+        }, red::kOneBlockPhase));
     } else {
         const double nm = 1 / std::sqrt(cosx * cosx + cosy * cosy);
         const double kx = k0 * cosx * nm, ky = k0 * cosy * nm;
@@ -1338,7 +1339,7 @@ int qsim_hip_born_xsection(qsim_born_job *j, int e, double cosx, double cosy, do
             const c128 t = (tot_at(idx, ix, iy, 0) * V[idx].x) * mk(cs, -sn);
             v[0] = t.x;
             v[1] = t.y;
-        }));
+        }, red::kOneBlockPhase));
     }
     const qsim_c128 r{rs[0], rs[1]};
     const cd rr(r.re, r.im);

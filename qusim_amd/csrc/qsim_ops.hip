@@ -599,7 +599,7 @@ int qsim_hip_abs2_k2d(const qsim_c128 *a_, double ax, size_t nx, double ay, size
     return reduce_sum<1>(n, s, out, [=] __device__(size_t idx, double *v) {
         double i = (double)fold_half(idx / ny, nx), j = (double)fold_half(idx % ny, ny);
         v[0] = abs2(a[idx]) * (i * i * ax + j * j * ay);
-    });
+    }, kOneBlockDiv);
 }
 
 int qsim_hip_abs2_k3d(const qsim_c128 *a_, double ax, size_t nx, double ay, size_t ny,
@@ -614,7 +614,7 @@ int qsim_hip_abs2_k3d(const qsim_c128 *a_, double ax, size_t nx, double ay, size
         double fk = (double)fold_half(k, nz), fj = (double)fold_half(r % ny, ny),
                fi = (double)fold_half(r / ny, nx);
         v[0] = abs2(a[idx]) * (fi * fi * ax + fj * fj * ay + fk * fk * az);
-    });
+    }, kOneBlockDiv);
 }
 
 int qsim_hip_abs2_mul_real(const qsim_c128 *a_, const double *V, size_t n, double *out,
@@ -668,7 +668,7 @@ int qsim_hip_xsection3d(const qsim_c128 *psi0_, const qsim_c128 *psi_, const qsi
         c128 t = ((psi0[idx] + psi[idx]) * V[idx].x) * mk(cs, sn);
         v[0] = t.x;
         v[1] = t.y;
-    }));
+    }, kOneBlockPhase));
     out->re = r[0];
     out->im = r[1];
     return QSIM_OK;
@@ -695,7 +695,7 @@ int qsim_hip_xsection2d(const qsim_c128 *psi0_, const qsim_c128 *psi_, const qsi
         c128 t = ((psi0[idx] + psi[idx]) * V[idx].x) * mk(cs, -sn);
         v[0] = t.x;
         v[1] = t.y;
-    }));
+    }, kOneBlockPhase));
     out->re = r[0];
     out->im = r[1];
     return QSIM_OK;

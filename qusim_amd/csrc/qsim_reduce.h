@@ -3,8 +3,7 @@
 // partial sums live in the per-device scratch block (no allocation per
 // call); the last kernel writes the result to pinned host memory, and the
 // host waits for the stream.  (A copy command in between cost 6 to 8 us a
-// call; arrays of up to kOneBlock elements take one workgroup and one
-// launch: a norm of 256 points 15.1 -> 7.3 us.)
+// call; short arrays take one workgroup and one launch, kOneBlock.)
 #pragma once
 
 #include <cstring>
@@ -15,7 +14,15 @@ namespace qsim {
 namespace red {
 
 constexpr int kBlock = 256;
-constexpr size_t kOneBlock = 4096;   // 16 elements a thread
+// The longest array that one workgroup reduces in one launch, by what an
+// element costs it.  Two launches take the same time up to 8000 elements, one
+// grows with them; us a call, 256 elements, at the limit, and two launches
+// there: norm 13.5, 15.4, 17.4; kinetic energy in 3D (64-bit divisions of the
+// index) 14.3, 17.6, 17.6; 3D cross section (and a sine and cosine) 16.0, 19.4,
+// 19.4 (with 4096 for all 25.6).
+constexpr size_t kOneBlock = 4096;
+constexpr size_t kOneBlockDiv = 2560;
+constexpr size_t kOneBlockPhase = 1536;
 
 template <typename F>
 __global__ void __launch_bounds__(kBlock) k_map(size_t n, F f)
@@ -129,9 +136,9 @@ __global__ void __launch_bounds__(kBlock) k_reduce_sum_final(int nb, const dd *p
 }
 
 template <int K, typename F>
-int reduce_sum(size_t n, qsim_stream_t s, double *host_out, F f)
+int reduce_sum(size_t n, qsim_stream_t s, double *host_out, F f, size_t one_block = kOneBlock)
 {
-    size_t nb = n <= kOneBlock ? 1 : grid_for(n);
+    size_t nb = n <= one_block ? 1 : grid_for(n);
     Scratch sc;
     QSIM_TRY(scratch_acquire(nb * K * sizeof(dd), &sc));
     dd *partial = reinterpret_cast<dd *>(sc.dev);
@@ -199,9 +206,10 @@ __global__ void __launch_bounds__(kBlock) k_reduce_ext_final(int nb, const doubl
 }
 
 template <bool MAX, typename F>
-int reduce_ext(size_t n, qsim_stream_t s, double init, double *host_out, F f)
+int reduce_ext(size_t n, qsim_stream_t s, double init, double *host_out, F f,
+               size_t one_block = kOneBlock)
 {
-    size_t nb = n <= kOneBlock ? 1 : grid_for(n);
+    size_t nb = n <= one_block ? 1 : grid_for(n);
     Scratch sc;
     QSIM_TRY(scratch_acquire(nb * sizeof(double), &sc));
     double *partial = reinterpret_cast<double *>(sc.dev);

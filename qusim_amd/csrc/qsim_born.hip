@@ -16,9 +16,9 @@
 //   outer sweep (axis 0, strided lines): FFT_x, G0 multiply, IFFT_x.
 // psi0 = e^{i k.r} and the absorbing layer (src/Perburbation.h:150-177) are
 // separable, so both come from per-axis tables instead of grid arrays; the
-// physical V is stored once for all energies.  Grids whose axes are composite
-// lengths with prime factors of at most 13 run the same passes on mixed-radix
-// lines (qsim_mix_born.hip, complex128); other grids the reference's order.
+// physical V is stored once for all energies.  Other grids whose axes mix_plan
+// takes (qsim_mix.h) run the same passes on mixed-radix lines
+// (qsim_mix_born.hip, complex128); the rest the reference's order.
 //
 // Precision 64: complex128 iterates.  Precision 32: complex64 iterates with
 // FP64 V, FP64 phase/absorber tables and FP64 residual sums.

@@ -25,7 +25,7 @@ struct BornDev {
     double E, eps, slow, inv_n;
     double inv_eps;        // 1 / eps (0 when eps is 0)
     double a[3];           // (2 pi hbar / (d n))^2 / 2m per axis
-    double *resid;         // per-block residual partial sums [2 * nblocks]
+    double *resid;         // residual partial sums: 2 per block, on mixed-radix grids 4
 };
 
 // potential with the absorbing layer, in the reference's summation order

@@ -1,10 +1,10 @@
 // qsim_fft.hip -- FourierTransform{1,2,3}D plans on gfx950 (replaces the
 // cuFFT Z2Z plans of src/FourierTransform.cpp:84-128, 336-360, 495-519 and
 // the KISS/FFTW CPU transforms).  Power-of-two axes up to 4096 (FP64) / 8192
-// (FP32) run the register-resident Stockham kernel; composite lengths up to
-// 5120 with prime factors of at most 13 run the mixed-radix kernel
-// (qsim_mix_fft.hip); every other length that fits twice in LDS runs the
-// generic kernel.
+// (FP32) run the register-resident Stockham kernel; the lengths that mix_plan
+// takes (qsim_mix.h) the mixed-radix kernel (qsim_mix_fft.hip); every other
+// length that fits twice in LDS the generic kernel; longer powers of two, as
+// the innermost axis, two four-step passes.
 #include <cmath>
 #include <map>
 #include <mutex>

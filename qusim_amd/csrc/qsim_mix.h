@@ -1,10 +1,10 @@
 // qsim_mix.h -- mixed-radix line transforms for lengths that are not a power
 // of two (and for the short powers of two that have no fused kernel).
 //
-// A length n whose prime factors are at most 13 is split at plan time into
-// 2..6 radices of at most 16 (MixPlan); the kernels switch on the radix of
-// each Stockham pass at run time, so one compiled kernel serves every such
-// length.  A workgroup holds L lines (a power of two) in LDS, element m of
+// mix_plan states which lengths run here.  It splits a length into 2..6
+// radices of at most 15, with a pass of paired sums for each prime above 13
+// (MixPlan); the kernels switch on the radix of each Stockham pass at run
+// time, so one compiled kernel serves every such length.  A workgroup holds L lines (a power of two) in LDS, element m of
 // line l at slot(m * L + l): lanes run over the lines first, so the
 // exchanges of 4 or more lines touch whole 64-128 B runs whatever the radix,
 // global loads of strided lines are coalesced, and the line index is a mask
@@ -421,7 +421,8 @@ struct MixDft<15> {
 // where it is used (the table stays in LDS).  With w^4 + q and w^8 + q as
 // products of two entries 1000 points cost 315 us instead of 333 (O4, 20 steps),
 // but after 60 transform pairs (on the CPU, 51 lengths, the same inputs) the
-// error was 1.36 times that of direct sums in the mean instead of 1.19.
+// error was 1.36 times that of direct sums in the mean instead of 1.19 (all
+// with the butterflies' constants still rounded once).
 template <int R>
 struct MixTw {
     const c128 *t;
@@ -758,7 +759,9 @@ __device__ __forceinline__ void mix_two(MixWg<T> &w, const MixPlan &p, In in, Pr
 // instructions of its butterflies, 4 cycles each on one of 4 SIMDs.  The fixed
 // part is fitted: 300, 700 and 1800 cycles make 4, 4 and 3 passes of a
 // 1000-point line held alone (5.3, 5.3 and 5.7 us a step), 3, 2 and 2 of 360
-// points (4.2, 3.8 and 3.8), and differ by less than 5% on grids.
+// points (4.2, 3.8 and 3.8), and differ by less than 5% on grids (timed without
+// the low parts; 1000 and 360 points take 6.1 and 4.6 us with them, of which the
+// host's call is a part).
 inline double mix_cost(int R, double work)
 {
     // butterfly, twiddles and index arithmetic; of the low parts' instructions
@@ -794,11 +797,13 @@ inline void mix_split(int n, int maxr, int depth, double work, double cost, int 
         }
 }
 
-// `work`: line elements that a CU holds at a time.  false when n is not a
-// composite number with prime factors of at most 13, 4 <= n <= kMixMaxLen, or
-// any number with a larger prime factor whose line fits LDS twice (mix_fits:
-// up to 3150 points).  *out is then an empty plan (n = 0): callers keep it as
-// "no mixed-radix line here".
+// The lengths of mixed-radix lines: composite numbers with prime factors of at
+// most 13 from 4 to kMixMaxLen, and numbers with a larger prime factor, primes
+// included, while the twiddles and two lines fit 160 KiB (mix_fits: every one
+// up to 3150).  Not among them: 1 to 3, the primes 5 to 13, and from 3151 on
+// most lengths with a prime factor above 13.  false for those, and *out is an
+// empty plan (n = 0), which callers keep as "no mixed-radix line here".  `work`:
+// line elements that a CU holds at a time.
 bool mix_fits(const MixPlan &p);
 inline bool mix_plan(size_t n, double work, MixPlan *out)
 {

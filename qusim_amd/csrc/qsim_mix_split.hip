@@ -12,9 +12,11 @@ namespace qsim {
 constexpr int kMix1dThreads = 768;
 
 // Lines are read once a sweep: from 6 MiB a sweep on, non-temporal loads keep
-// E_V and the tables in L2 (1000 x 1000: 34.0 -> 32.5 us a step, 1200 x
-// 1200 61.8 -> 60.4, both timed with two entries' products as higher twiddle
-// powers; 300 x 300 would lose 4%).
+// E_V and the tables in L2.  us a step with plain and with non-temporal loads:
+// 300 x 300 (1.4 MiB) 17.0 and 18.0, 500 x 500 (3.8) 21.4 and 21.7, 600 x 600
+// (5.5) 24.4 and 24.5, 640 x 660 (6.4) 26.7 and 26.6, 700 x 700 (7.5) 28.3 and
+// 27.8, 900 x 900 32.8 and 30.4, 1000 x 1000 35.5 and 31.9, 1500 x 1500 81.7 and
+// 80.6.
 template <bool NT>
 __device__ __forceinline__ c128 ld_psi(const c128 *p)
 {
@@ -28,11 +30,10 @@ static bool psi_nt(const MixPlan &p, size_t nlines)
 
 // Row and column sweeps: 32 B of psi and 16 B of E_V per point move once.  At
 // 1000 x 1000 a step takes 32 us (the unfused order's 8 passes: 300 us) and at
-// 1500 x 1500 82 us (2.2 TB/s of the 80 B);
-// below that the chain of one workgroup's passes bounds the sweeps (750 x 600:
-// 27 us a step, waves wait for 77% of their cycles in the row sweep and 62% in
-// the column sweep), above it the LDS
-// exchanges.
+// 1500 x 1500 80 us (2.2 TB/s of the 80 B); below that the chain of one
+// workgroup's passes bounds the sweeps (750 x 600: 28 us a step, waves wait for
+// 76% of their cycles in the row sweep and 65% in the column sweep), above it
+// the LDS exchanges.
 template <int MODE, bool NT>
 __global__ void __launch_bounds__(kMixMaxThreads)
     k_mix_row(c128 *psi, const c128 *ev, int twice, unsigned nrows, MixPlan p, MixDims d,
@@ -103,7 +104,7 @@ __global__ void __launch_bounds__(kMixMaxThreads)
 // All steps of one line: 768 threads at most, so that 168 registers are left (at
 // 128 the wide radices spilled: 1000 points 6.2 against 5.3 us a step when
 // timed).  Bound by the latency of its passes: a step of n = 1000 is 6 of about
-// 0.9 us (an O4 stage 5.6 us); the unfused order's 7 launches took 66 us.
+// 1 us (an O4 stage 6.0 us); the unfused order's 7 launches took 66 us.
 __global__ void __launch_bounds__(kMix1dThreads)
     k_mix_1d(SplitDev J, Prog1D prog, size_t nsteps, double scale, double scale_lo,
              MixPlan p, MixDims d, int nreal, const c128 *__restrict__ tw)

@@ -11,10 +11,10 @@
 // with E_T = Tx Ty separable and 1/(nx ny) folded into Tx.  The first sweep
 // only applies E_V then FFT_y; the last only IFFT_y then E_V.
 // 1D (power-of-two): one workgroup per job keeps psi in registers for all
-// steps.  Composite lengths with prime factors of at most 13 run the same
-// schedule on mixed-radix lines (qsim_mix_split.hip), the infinite wall as its
-// odd extension; other sizes run the reference's op sequence unfused (FFT
-// plans + pointwise kernels).
+// steps.  Other lengths that mix_plan takes (qsim_mix.h) run the same schedule
+// on mixed-radix lines (qsim_mix_split.hip), the infinite wall as its odd
+// extension of twice the points; the rest run the reference's op sequence
+// unfused (FFT plans + pointwise kernels).
 //
 // Precision 64: complex128 everywhere.  Precision 32 (FP32-mixed): psi is
 // stored and transformed in complex64; every phase factor and inter-pass
